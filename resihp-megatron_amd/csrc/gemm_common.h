@@ -7,8 +7,8 @@
 #include <atomic>
 #include <string>
 
+#include "dma.h"
 #include "fp8_common.h"
-#include "rhp_common.h"
 
 
 namespace rhp {
@@ -1175,29 +1175,6 @@ __device__ __forceinline__ void interleave_reads() {
     }
 }
 
-
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-
-struct Rsrc {
-    i32x4_t d;
-};
-__device__ __forceinline__ Rsrc make_dma_rsrc(const void* base, int64_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(base);
-    Rsrc r;
-    r.d[0] = __builtin_amdgcn_readfirstlane(static_cast<int>(a));
-    r.d[1] = __builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32));
-    r.d[2] = __builtin_amdgcn_readfirstlane(static_cast<int>(bytes > 0x7ffffff0 ? 0x7ffffff0 : bytes));
-    r.d[3] = 0x00020000;
-    return r;
-}
-// 16 bytes per lane from the buffer at voff + soff into LDS at lds + 16 * lane.
-__device__ __forceinline__ void dma16(const Rsrc& r, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :
-                 : "v"(voff), "s"(r.d), "s"(__builtin_amdgcn_readfirstlane(soff)),
-                   "s"(__builtin_amdgcn_readfirstlane(lds))
-                 : "memory");
-}
 
 // Wait until every load this wave issued has landed.
 __device__ __forceinline__ void wait_loads_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }

@@ -13,8 +13,9 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
-#include "rhp_common.h"
+#include "dma.h"
 
 namespace rhp {
 namespace {
@@ -72,81 +73,117 @@ template <class AT> __device__ __forceinline__ bool better(AT va, int ia, AT vb,
     return va > vb || (va == vb && ia < ib);
 }
 
+// v of the lane a DPP control picks (every lane takes part).
+template <int CTRL> __device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL> __device__ __forceinline__ double dpp(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// Largest v of each aligned group of lpt lanes (a power of two), no NaN among
+// them, in every lane of the group: lane exchanges within 16 lanes are DPP
+// (quad swaps, then mirrored halves, whose lanes already agree).
+template <class AT> __device__ __forceinline__ AT group_max(AT v, int lpt) {
+    auto take = [&](AT o) { v = o > v ? o : v; };
+    if (lpt > 1) take(dpp<0xB1>(v));    // quad_perm 1 0 3 2
+    if (lpt > 2) take(dpp<0x4E>(v));    // quad_perm 2 3 0 1
+    if (lpt > 4) take(dpp<0x141>(v));   // row_half_mirror
+    if (lpt > 8) take(dpp<0x140>(v));   // row_mirror
+    if (lpt > 16) take(__shfl_xor(v, 16, 64));
+    if (lpt > 32) take(__shfl_xor(v, 32, 64));
+    return v;
+}
+
 // Selection and gates of a block's tb tokens (first token t_block) from their
-// logits lg[tb][E] in LDS; sel[tb][k] is LDS scratch.  nthreads: block size.
+// logits in LDS, token tl's at lg + tl ld; sel[tb][k] and num[tb][k] are LDS
+// scratch.  nthreads: block size.
+//   A group of lpt lanes selects a token's experts: the largest remaining key
+// by lane exchange, its expert by a ballot (ties, rare, by a second pass over
+// the ids).  Exchanging (key, id) pairs through LDS shuffles took 52 of 120 us
+// at 16384 tokens, 64 experts, top 6.  A lane keeps the keys of its first two
+// experts (all of them up to 128 experts) in registers.
+//   Gates: one thread per (token, slot); sums in slot order.
 template <class AT>
-__device__ __forceinline__ void select_and_gate(const AT* lg, int* sel, int64_t t_block, int tb, int nthreads,
-                                                int64_t T, int E, int k, int score, int normalize, AT scale,
-                                                const AT* __restrict__ bias, int32_t* __restrict__ topi,
+__device__ __forceinline__ void select_and_gate(const AT* lg, int ld, int* sel, AT* num, int64_t t_block, int tb,
+                                                int nthreads, int64_t T, int E, int k, int score, int normalize,
+                                                AT scale, const AT* __restrict__ bias, int32_t* __restrict__ topi,
                                                 AT* __restrict__ gates) {
     const int tid = threadIdx.x;
-    // Top-k by wavefront shuffles.  A group of lpt lanes handles one
-    // token; each lane owns experts lane_in_group + c * lpt.
     int lpt = 1;
     while (lpt < E && lpt < 64) lpt <<= 1;
     const int lane = tid & 63, wave = tid >> 6;
     const int gl = lane & (lpt - 1);
     const int groups_per_block = (nthreads / 64) * (64 / lpt);
     const int my_group = wave * (64 / lpt) + lane / lpt;
-    const int cand = (E + lpt - 1) / lpt;
+    const int cand = (E + lpt - 1) / lpt;   // each lane owns experts gl + c * lpt
+    const int none = 0x7fffffff;
+    const uint64_t group_lanes = (lpt == 64 ? ~0ull : (1ull << lpt) - 1) << (lane & ~(lpt - 1));
     for (int tl0 = 0; tl0 < tb; tl0 += groups_per_block) {
         const int tl = tl0 + my_group;
         const bool active = tl < tb && (t_block + tl) < T;
+        auto key = [&](int c) {
+            const int e = gl + c * lpt;
+            if (!active || e >= E) return neg_inf<AT>();
+            AT v = lg[tl * ld + e];
+            if (score == RHP_SCORE_SIGMOID) v = rhp_sigmoid(v);
+            if (bias) v = v + bias[e];
+            return v != v ? neg_inf<AT>() : v;
+        };
+        const AT key0 = key(0), key1 = cand > 1 ? key(1) : neg_inf<AT>();
         uint32_t taken = 0;   // bit c: candidate c already chosen (cand <= 16 since E <= 1024)
         for (int j = 0; j < k; ++j) {
             AT bv = neg_inf<AT>();
-            int bi = 0x7fffffff;
+            int bi = none;
             if (active) {
                 for (int c = 0; c < cand; ++c) {
                     const int e = gl + c * lpt;
                     if (e >= E || ((taken >> c) & 1u)) continue;
-                    AT v = lg[static_cast<size_t>(tl) * E + e];
-                    if (score == RHP_SCORE_SIGMOID) v = rhp_sigmoid(v);
-                    if (bias) v = v + bias[e];
-                    if (v != v) v = neg_inf<AT>();
+                    const AT v = c == 0 ? key0 : c == 1 ? key1 : key(c);
                     if (better(v, e, bv, bi)) { bv = v; bi = e; }
                 }
             }
-            for (int o = lpt >> 1; o >= 1; o >>= 1) {
-                AT ov = __shfl_xor(bv, o, 64);
-                int oi = __shfl_xor(bi, o, 64);
-                if (better(ov, oi, bv, bi)) { bv = ov; bi = oi; }
+            const AT m = group_max(bv, lpt);
+            uint64_t win = __ballot(bi != none && bv == m) & group_lanes;
+            int id = bi;
+            if (__ballot(__popcll(win) > 1)) {   // a tie in some group of the wave: its lowest id
+                int low = bi != none && bv == m ? bi : none;
+                for (int o = lpt >> 1; o >= 1; o >>= 1) low = min(low, __shfl_xor(low, o, 64));
+                id = low;
             }
-            if (active) {
-                if ((bi & (lpt - 1)) == gl) taken |= 1u << (bi / lpt);
-                if (gl == 0) sel[tl * k + j] = bi;
+            if (active && bi == id && ((win >> lane) & 1)) {
+                taken |= 1u << (id / lpt);
+                sel[tl * k + j] = id;
             }
         }
     }
     __syncthreads();
 
-    // Gates, one thread per token, sums in slot order.
-    for (int tl = tid; tl < tb; tl += nthreads) {
-        const int64_t t = t_block + tl;
-        if (t >= T) continue;
-        const AT* l = lg + static_cast<size_t>(tl) * E;
+    // num: the slot's exp (softmax, over the selected logits) or sigmoid.
+    const int n = static_cast<int>(min<int64_t>(tb, T - t_block)) * k;
+    for (int i = tid; i < n; i += nthreads) {
+        const int tl = i / k;
+        const AT* l = lg + tl * ld;
         const int* s = sel + tl * k;
-        AT g[kMaxTopK];
-        AT sum = AT(0);
+        const AT v = l[s[i - tl * k]];
         if (score == RHP_SCORE_SOFTMAX) {
             AT m = l[s[0]];
             for (int j = 1; j < k; ++j) m = (l[s[j]] > m) ? l[s[j]] : m;
-            for (int j = 0; j < k; ++j) {
-                g[j] = rhp_exp_t(l[s[j]] - m);
-                sum = (j == 0) ? g[j] : sum + g[j];
-            }
-            for (int j = 0; j < k; ++j) g[j] = (g[j] / sum) * scale;
+            num[i] = rhp_exp_t(v - m);
         } else {
-            for (int j = 0; j < k; ++j) {
-                g[j] = rhp_sigmoid(l[s[j]]);
-                sum = (j == 0) ? g[j] : sum + g[j];
-            }
-            for (int j = 0; j < k; ++j) g[j] = (normalize ? g[j] / sum : g[j]) * scale;
+            num[i] = rhp_sigmoid(v);
         }
-        for (int j = 0; j < k; ++j) {
-            topi[t * k + j] = s[j];
-            gates[t * k + j] = g[j];
-        }
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += nthreads) {
+        const AT* g = num + i / k * k;
+        AT sum = g[0];
+        for (int j = 1; j < k; ++j) sum = sum + g[j];
+        const AT v = num[i];
+        topi[t_block * k + i] = sel[i];
+        gates[t_block * k + i] = (score == RHP_SCORE_SOFTMAX || normalize ? v / sum : v) * scale;
     }
 }
 
@@ -159,7 +196,8 @@ __global__ __launch_bounds__(kThreads) void route_kernel(const XT* __restrict__ 
     extern __shared__ __align__(16) unsigned char smem_raw[];
     AT* part = reinterpret_cast<AT*>(smem_raw);                 // [tb][S][E]
     AT* lg = part + static_cast<size_t>(rs.tb) * rs.S * E;      // [tb][E]
-    int* sel = reinterpret_cast<int*>(lg + static_cast<size_t>(rs.tb) * E);   // [tb][k]
+    AT* num = lg + static_cast<size_t>(rs.tb) * E;              // [tb][k]
+    int* sel = reinterpret_cast<int*>(num + rs.tb * k);         // [tb][k]
 
     const int tid = threadIdx.x;
     const int64_t t_block = static_cast<int64_t>(blockIdx.x) * rs.tb;
@@ -219,122 +257,172 @@ __global__ __launch_bounds__(kThreads) void route_kernel(const XT* __restrict__ 
     }
     __syncthreads();
 
-    select_and_gate<AT>(lg, sel, t_block, rs.tb, kThreads, T, E, k, score, normalize, scale, bias, topi, gates);
+    select_and_gate<AT>(lg, E, sel, num, t_block, rs.tb, kThreads, T, E, k, score, normalize, scale, bias, topi, gates);
 }
 
-// Router logits of bfloat16 tokens, the production path.  One lane per token
-// (64 tokens per block): every lane of a wave runs the same chains, so the
-// router weights it multiplies by are wave-uniform and come through scalar
-// loads, while each lane streams its own token row in whole 128-byte lines.
-// Work is split over the block's waves one of two ways:
-//   segment mode (few experts): wave w takes segments w, w + nw, ... of each
-//     group of EC experts; the segment chains go to LDS and are then added
-//     left to right;
-//   expert mode (many experts): wave w takes expert groups w, w + nw, ... and
-//     runs their segments in order, adding each finished chain to the running
-//     total in registers.
-// Either way every logit is the same fma chains summed in the same order as
-// route_kernel's (and the oracle's), bit for bit.  Experts past E in the last
-// group are computed on a clamped row and discarded.  TOK tokens per block:
-// 64, or 32 where 64-token blocks would not reach every CU (lanes 32..63 then
-// repeat lanes 0..31's rows, which keeps the loads and weights wave-uniform,
-// and store nothing).
-constexpr int kRtTokens = 64;
-constexpr int kRtMaxWaves = 16;
+// Router logits of bfloat16 and float32 tokens on the matrix cores, the
+// production path.  v_mfma_f32_16x16x4_f32 adds its four products one after
+// the other, each a correctly rounded fused multiply-add with subnormals
+// (compared with fmaf chains bit for bit on random, subnormal, widely spread
+// and NaN / infinite inputs).  So the logits are the very chains of
+// route_kernel and the oracle, bit for bit.  (The one-k shapes are exact too,
+// at a quarter of the rate.)  A wave's task is 16 experts by TI x 16 tokens by
+// four 256-element segments, whose chains are independent.
+//
+// Each wave streams its rows through LDS of its own, 16 elements of every row
+// a batch, NB batches deep, with direct HBM -> LDS loads: read straight into
+// registers, every lane's 16 bytes were a cache line of their own and the
+// loads' address rate bound the kernel.  No barrier until the chains are
+// complete; the chains of a round of tasks then meet in LDS (over the staging
+// buffers) and are added left to right.
+//   Measured (64 experts, 2048 inputs, top 6; a lane per token on the VALU
+// before): 64 tokens 144 -> 26 us, 4096 tokens 165 -> 30, 16384 206 -> 96;
+// 4096 tokens by 128 experts, top 8: 328 -> 51; 1000 float32 tokens by 8
+// experts, 1024 inputs: 99 -> 14.  What bounds it now: up to 4096 tokens the
+// chain of one task (256 MFMAs a wave, two waves a SIMD) and the selection.
+constexpr int kRtBatch = 16;
+typedef float f32x4_route_t __attribute__((ext_vector_type(4)));
 
-// Chains of EC experts (rows wr) over one segment [i0, i0 + seg) of a token row.
-template <int EC>
-__device__ __forceinline__ void segment_chains(const bf16* xr, const float* const* wr, int i0, int seg, float* acc) {
-#pragma unroll
-    for (int b = 0; b < EC; ++b) acc[b] = 0.0f;
-    for (int g = 0; g < seg; g += 64) {
-        uint4 xv[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-            if (g + c * 8 < seg) xv[c] = *reinterpret_cast<const uint4*>(xr + i0 + g + c * 8);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (g + c * 8 >= seg) break;
-            const uint32_t q[4] = {xv[c].x, xv[c].y, xv[c].z, xv[c].w};
-            float xf[8];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                xf[2 * i] = __uint_as_float(q[i] << 16);
-                xf[2 * i + 1] = __uint_as_float(q[i] & 0xffff0000u);
-            }
-            const int i = i0 + g + c * 8;
-#pragma unroll
-            for (int ii = 0; ii < 8; ++ii)
-#pragma unroll
-                for (int b = 0; b < EC; ++b) acc[b] = fma_t(xf[ii], wr[b][i + ii], acc[b]);
-        }
-    }
-}
+// Staged rows of a 64-row tile (16 rows by 4 segments): C chunks of 16 bytes
+// a row, chunk c of row p at c ^ (p / (16 / C) mod C), so that the 16 rows of a
+// ds_read_b128 hit distinct banks.
+template <int C> __device__ __forceinline__ int rt_chunk(int p, int c) { return c ^ ((p / (16 / C)) & (C - 1)); }
 
-template <int EC, int TOK>
-__global__ __launch_bounds__(64 * kRtMaxWaves) void route_bf16_kernel(const bf16* __restrict__ x,
-                                                                    const float* __restrict__ w,
-                                                                    const float* __restrict__ bias, int64_t T, int h,
-                                                                    int E, int k, int score, int normalize, float scale,
-                                                                    int seg, int S, int expert_mode,
-                                                                    float* __restrict__ logits,
-                                                                    int32_t* __restrict__ topi,
-                                                                    float* __restrict__ gates) {
+template <class XT, int TI, int W, int NB>
+__global__ __launch_bounds__(64 * W) void route_mfma_kernel(const XT* __restrict__ x, const float* __restrict__ w,
+                                                            const float* __restrict__ bias, int64_t T, int h, int E,
+                                                            int k, int score, int normalize, float scale, int seg,
+                                                            int S, float* __restrict__ logits,
+                                                            int32_t* __restrict__ topi, float* __restrict__ gates) {
+    constexpr int TB = 16 * TI;
+    constexpr int XC = kRtBatch * static_cast<int>(sizeof(XT)) / 16, WC = kRtBatch * 4 / 16;   // chunks per staged row
+    constexpr int kBufBytes = 1024 * (WC + XC * TI), kLoads = WC + XC * TI;
+    __shared__ __align__(1024) uint8_t stage[W * NB * kBufBytes];
+    static_assert(W * 4 * 16 * TB * 4 <= W * NB * kBufBytes, "a round's chains fit over the staging buffers");
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    float* lg = reinterpret_cast<float*>(smem_raw);                           // [TOK][E]
-    int* sel = reinterpret_cast<int*>(lg + static_cast<size_t>(TOK) * E);     // [TOK][k]
-    float* part = reinterpret_cast<float*>(sel + TOK * k);                    // [S][EC][TOK], segment mode
-    const int lane = threadIdx.x & 63, tl = lane % TOK;
-    const bool owner = lane < TOK;
+    const int ld = E | 1;                                   // odd row pitch: no bank conflicts
+    float* lg = reinterpret_cast<float*>(smem_raw);         // [TB][ld]
+    float* num = lg + TB * ld;                              // [TB][k]
+    int* sel = reinterpret_cast<int*>(num + TB * k);        // [TB][k]
+    float* part = reinterpret_cast<float*>(stage);          // [tasks][4 segments][16 experts][TB]
+    const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int nw = blockDim.x >> 6;
-    const int64_t t_block = static_cast<int64_t>(blockIdx.x) * TOK;
-    const int64_t t = t_block + tl < T ? t_block + tl : t_block;   // lanes past T repeat a valid row
-    const bf16* xr = x + t * h;
-    if (expert_mode) {
-        for (int e0 = wave * EC; e0 < E; e0 += nw * EC) {
-            const float* wr[EC];
+    const int64_t t_block = static_cast<int64_t>(blockIdx.x) * TB;
+    const int tb = static_cast<int>(min<int64_t>(TB, T - t_block));
+    const Rsrc rw = make_dma_rsrc(w, static_cast<int64_t>(E) * h * 4);
+    const Rsrc rx = make_dma_rsrc(x + t_block * h, static_cast<int64_t>(tb) * h * sizeof(XT));
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(stage)) + wave * NB * kBufBytes;
+    const uint8_t* mine = stage + wave * NB * kBufBytes;
+    // A round: ge expert tiles by nq segment quads, one task a wave.
+    const int n_sq = (S + 3) / 4, n_et = (E + 15) / 16;
+    const int nq = min(n_sq, W), ge = max(1, W / n_sq);
+    for (int et0 = 0; et0 < n_et; et0 += ge)
+        for (int sq0 = 0; sq0 < n_sq; sq0 += nq) {
+            const int tasks = min(ge, n_et - et0) * min(nq, n_sq - sq0), n_q = min(nq, n_sq - sq0);
+            f32x4_route_t acc[TI][4];   // [token tile][segment]: tokens 4 q .. + 3 of expert r
 #pragma unroll
-            for (int b = 0; b < EC; ++b) wr[b] = w + static_cast<int64_t>(min(e0 + b, E - 1)) * h;
-            float total[EC], acc[EC];
-            for (int s = 0; s < S; ++s) {
-                segment_chains<EC>(xr, wr, s * seg, seg, acc);
+            for (int t = 0; t < TI; ++t)
 #pragma unroll
-                for (int b = 0; b < EC; ++b) total[b] = s == 0 ? acc[b] : total[b] + acc[b];
-            }
+                for (int b = 0; b < 4; ++b) acc[t][b] = f32x4_route_t{};
+            if (wave < tasks) {
+                const int e0 = (et0 + wave / n_q) * 16, s0 = 4 * (sq0 + wave % n_q);
+                // Byte offsets of the pieces this lane loads; rows past the last expert, token or segment
+                // repeat a valid one, and their results are dropped.
+                uint32_t ow[WC], ox[TI][XC];
 #pragma unroll
-            for (int b = 0; b < EC; ++b)
-                if (owner && e0 + b < E) lg[tl * E + e0 + b] = total[b];
-        }
-        __syncthreads();
-    } else {
-        for (int e0 = 0; e0 < E; e0 += EC) {
-            const float* wr[EC];
+                for (int j = 0; j < WC; ++j) {
+                    const int p = (j * 64 + lane) / WC, c = rt_chunk<WC>(p, lane % WC);
+                    ow[j] = (static_cast<uint32_t>(min(e0 + p % 16, E - 1)) * h + min(s0 + p / 16, S - 1) * seg) * 4u + c * 16u;
+                }
 #pragma unroll
-            for (int b = 0; b < EC; ++b) wr[b] = w + static_cast<int64_t>(min(e0 + b, E - 1)) * h;
-            for (int s = wave; s < S; s += nw) {
-                float acc[EC];
-                segment_chains<EC>(xr, wr, s * seg, seg, acc);
+                for (int t = 0; t < TI; ++t)
 #pragma unroll
-                for (int b = 0; b < EC; ++b)
-                    if (owner) part[(s * EC + b) * TOK + tl] = acc[b];
-            }
-            __syncthreads();
-            for (int idx = threadIdx.x; idx < EC * TOK; idx += blockDim.x) {
-                const int b = idx / TOK, r = idx % TOK;
-                if (e0 + b < E) {
-                    float total = part[b * TOK + r];
-                    for (int s = 1; s < S; ++s) total = total + part[(s * EC + b) * TOK + r];
-                    lg[r * E + e0 + b] = total;
+                    for (int j = 0; j < XC; ++j) {
+                        const int p = (j * 64 + lane) / XC, c = rt_chunk<XC>(p, lane % XC);
+                        ox[t][j] = (static_cast<uint32_t>(min(16 * t + p % 16, tb - 1)) * h + min(s0 + p / 16, S - 1) * seg) *
+                                       static_cast<uint32_t>(sizeof(XT)) + c * 16u;
+                    }
+                auto issue = [&](int b) {   // the loads of batch b into its buffer
+                    const uint32_t at = lds0 + (b % NB) * kBufBytes, i = static_cast<uint32_t>(b) * kRtBatch;
+#pragma unroll
+                    for (int j = 0; j < WC; ++j) dma16(rw, ow[j], i * 4, at + j * 1024);
+#pragma unroll
+                    for (int t = 0; t < TI; ++t)
+#pragma unroll
+                        for (int j = 0; j < XC; ++j)
+                            dma16(rx, ox[t][j], i * static_cast<uint32_t>(sizeof(XT)), at + (WC + t * XC + j) * 1024);
+                };
+                const int nb = (seg + kRtBatch - 1) / kRtBatch;
+#pragma unroll
+                for (int b = 0; b < NB - 1; ++b)
+                    if (b < nb) issue(b);
+                for (int b = 0; b < nb; ++b) {
+                    if (b + NB - 1 < nb) {
+                        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): batch b - 1 has been read from its buffer
+                        issue(b + NB - 1);
+                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 1) * kLoads) : "memory");
+                    } else if (NB > 2 && b + 1 < nb) {
+                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * kLoads) : "memory");
+                    } else {
+                        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                    }
+                    const uint8_t* buf = mine + (b % NB) * kBufBytes;
+                    // Lane l holds element 4 i + q of row r of each 16-row tile (rows 16 seg .. + 15 of the
+                    // stage).  Every read of the batch is issued before the first MFMA waits for one.
+                    float wf[4][4], xf[TI][4][4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int sg = 0; sg < 4; ++sg) {
+                            const int p = 16 * sg + r;
+                            wf[i][sg] = *reinterpret_cast<const float*>(buf + (p * WC + rt_chunk<WC>(p, i)) * 16 + 4 * q);
+#pragma unroll
+                            for (int t = 0; t < TI; ++t) {
+                                const uint8_t* xt = buf + (WC + t * XC) * 1024;
+                                if constexpr (sizeof(XT) == 2)
+                                    xf[t][i][sg] = bf16_to_f32(*reinterpret_cast<const uint16_t*>(
+                                        xt + (p * XC + rt_chunk<XC>(p, i / 2)) * 16 + (i % 2) * 8 + 2 * q));
+                                else
+                                    xf[t][i][sg] =
+                                        *reinterpret_cast<const float*>(xt + (p * XC + rt_chunk<XC>(p, i)) * 16 + 4 * q);
+                            }
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if (i % 2 == 0 && b * kRtBatch + 4 * i >= seg) break;   // a segment shorter than 256 may end here
+#pragma unroll
+                        for (int sg = 0; sg < 4; ++sg)
+#pragma unroll
+                            for (int t = 0; t < TI; ++t)
+                                acc[t][sg] = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[t][i][sg], wf[i][sg], acc[t][sg], 0, 0, 0);
+                    }
                 }
             }
+            __syncthreads();   // every wave is done with its staging buffers
+            if (wave < tasks)
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+#pragma unroll
+                    for (int t = 0; t < TI; ++t)
+                        *reinterpret_cast<float4*>(part + ((wave * 4 + b) * 16 + r) * TB + 16 * t + 4 * q) =
+                            make_float4(acc[t][b][0], acc[t][b][1], acc[t][b][2], acc[t][b][3]);
             __syncthreads();
+            const int s_end = min(4 * n_q, S - 4 * sq0);   // segments of this round
+            for (int idx = threadIdx.x; idx < min(ge, n_et - et0) * 16 * TB; idx += 64 * W) {
+                const int tile = idx / (16 * TB), at = idx % (16 * TB), e = (et0 + tile) * 16 + at / TB;
+                if (e < E) {
+                    const float* pp = part + tile * n_q * 4 * 16 * TB + at;
+                    float* out = lg + (at % TB) * ld + e;
+                    float total = sq0 ? *out + pp[0] : pp[0];
+                    for (int s = 1; s < s_end; ++s) total = total + pp[s * 16 * TB];
+                    *out = total;
+                }
+            }
+            __syncthreads();   // the sums are read before the next round's loads land
         }
-    }
-    const int tb = static_cast<int>(min<int64_t>(TOK, T - t_block));
-    for (int idx = threadIdx.x; idx < tb * E; idx += blockDim.x) logits[t_block * E + idx] = lg[idx];
-    select_and_gate<float>(lg, sel, t_block, TOK, blockDim.x, T, E, k, score, normalize, scale, bias, topi,
-                           gates);
+    for (int idx = threadIdx.x; idx < tb * E; idx += 64 * W) logits[t_block * E + idx] = lg[(idx / E) * ld + idx % E];
+    select_and_gate<float>(lg, ld, sel, num, t_block, TB, 64 * W, T, E, k, score, normalize, scale, bias, topi, gates);
 }
 
 }  // namespace
@@ -625,43 +713,37 @@ __global__ __launch_bounds__(kThreads) void route_bwd_kernel(const AT* __restric
     }
 }
 
-// Routing of bfloat16 tokens: route_bf16_kernel, whenever its LDS fits in
-// 64 KB; 0 = launched (or nothing to do), 1 = not taken.
-int launch_route_bf16(const void* x, const void* w, const void* bias, int64_t T, int h, int E, int k, int score,
-                      int normalize, double scale, void* logits, int32_t* topi, void* gates, hipStream_t stream,
-                      int* status) {
-    const int seg = std::min(256, h), S = h / seg;
-    const int ec = E >= 64 ? 16 : 8;
-    const int n_ec = (E + ec - 1) / ec;
-    const int expert_mode = n_ec >= S ? 1 : 0;
-    // 32-token blocks where 64-token ones would leave CUs without a block.
-    int cus = 0, dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        cus = 0;
-    const int tok = (T + kRtTokens - 1) / kRtTokens < cus ? kRtTokens / 2 : kRtTokens;
-    const size_t smem = static_cast<size_t>(tok) * E * sizeof(float) + static_cast<size_t>(tok) * k * sizeof(int) +
-                        (expert_mode ? 0 : static_cast<size_t>(S) * ec * tok * sizeof(float));
-    if (smem > 64 * 1024) {
-        *status = 1;
-        return 0;
-    }
-    *status = 0;
-    if (T == 0) return 0;
-    const int nw = std::min(expert_mode ? n_ec : S, kRtMaxWaves);
-    const dim3 grid(static_cast<unsigned>((T + tok - 1) / tok)), block(64 * nw);
-    const bf16* xb = static_cast<const bf16*>(x);
-    const float* wf = static_cast<const float*>(w);
-    const float* bf = static_cast<const float*>(bias);
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, block, smem, stream, xb, wf, bf, T, h, E, k, score, normalize,
-                           static_cast<float>(scale), seg, S, expert_mode, static_cast<float*>(logits), topi,
-                           static_cast<float*>(gates));
+// LDS of a route_mfma_kernel block beside its staging buffers (logits and selection of its tokens), and
+// what the buffers of eight waves leave for it.
+constexpr size_t rt_lds(int tb, int E, int k) { return static_cast<size_t>(tb) * ((E | 1) + 2 * k) * 4; }
+template <class XT, int TI, int NB> constexpr size_t rt_room() {
+    return 163840 - 8 * NB * 1024 * (kRtBatch * 4 / 16 + kRtBatch * sizeof(XT) / 16 * TI);
+}
+// bfloat16 tokens from which a block takes 32: they stage the weights half as often, but 16-token blocks
+// are quicker until they fill the CUs twice (64 experts: 4096 tokens 37 against 54 us, 8192 both 57).
+constexpr int64_t kRtWideTokens = 8192;
+
+template <class XT, int TI, int NB>
+int launch_route_mfma(const void* x, const void* w, const void* bias, int64_t T, int h, int E, int k, int score,
+                      int normalize, double scale, void* logits, int32_t* topi, void* gates, hipStream_t stream) {
+    const int seg = std::min(256, h), S = h / seg, tasks = ((E + 15) / 16) * ((S + 3) / 4);
+    auto go = [&](auto kern, int waves) {
+        hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((T + 16 * TI - 1) / (16 * TI))), dim3(64 * waves),
+                           rt_lds(16 * TI, E, k), stream, static_cast<const XT*>(x), static_cast<const float*>(w),
+                           static_cast<const float*>(bias), T, h, E, k, score, normalize, static_cast<float>(scale),
+                           seg, S, static_cast<float*>(logits), topi, static_cast<float*>(gates));
     };
-    if (ec == 16)
-        tok == kRtTokens ? go(route_bf16_kernel<16, kRtTokens>) : go(route_bf16_kernel<16, kRtTokens / 2>);
-    else
-        tok == kRtTokens ? go(route_bf16_kernel<8, kRtTokens>) : go(route_bf16_kernel<8, kRtTokens / 2>);
-    return check_launch("route_bf16_kernel");
+    if (tasks <= 4) go(route_mfma_kernel<XT, TI, 4, NB>, 4);
+    else go(route_mfma_kernel<XT, TI, 8, NB>, 8);
+    return check_launch("route_mfma_kernel");
+}
+
+// Sizes of bfloat16 tokens that are taken whatever the per-thread kernel's LDS limit: those whose
+// logits and, with few experts, segment sums of one block of tokens fit in 64 KB.
+bool bf16_route_fits(int64_t T, int h, int E, int k) {
+    const int S = h / std::min(256, h), ec = E >= 64 ? 16 : 8, n_ec = (E + ec - 1) / ec;
+    const size_t tok = (T + 63) / 64 < device_cus() ? 32 : 64;
+    return tok * (E + k) * 4 + (n_ec >= S ? 0 : static_cast<size_t>(S) * ec * tok * 4) <= 64 * 1024;
 }
 
 template <class XT, class AT>
@@ -680,10 +762,25 @@ int launch_route(const void* x, const void* w, const void* bias, int64_t T, int 
     rs.ntg = ntg;
     rs.tb = ntg * kTpt;
     const size_t smem = static_cast<size_t>(rs.tb) * per_token;
-    RHP_REQUIRE(smem <= 48 * 1024, "rhp_route: hidden size x experts too large for one routing block");
+    constexpr bool bf = std::is_same<XT, bf16>::value;
+    RHP_REQUIRE(smem <= 48 * 1024 || (bf && bf16_route_fits(T, h, E, k)),
+                "rhp_route: hidden size x experts too large for one routing block");
     if (T == 0) return 0;
+    if constexpr (std::is_same<AT, float>::value) {
+        if (static_cast<int64_t>(E) * h * 4 < (int64_t(1) << 31)) {
+            if constexpr (bf) {
+                if (T >= kRtWideTokens && rt_lds(32, E, k) <= rt_room<XT, 2, 2>())
+                    return launch_route_mfma<XT, 2, 2>(x, w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates, stream);
+                if (rt_lds(16, E, k) <= rt_room<XT, 1, 3>())
+                    return launch_route_mfma<XT, 1, 3>(x, w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates, stream);
+            }
+            if (rt_lds(16, E, k) <= rt_room<XT, 1, 2>())
+                return launch_route_mfma<XT, 1, 2>(x, w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates, stream);
+        }
+    }
     const int64_t blocks = (T + rs.tb - 1) / rs.tb;
-    hipLaunchKernelGGL((route_kernel<XT, AT>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads), smem, stream,
+    hipLaunchKernelGGL((route_kernel<XT, AT>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads),
+                       smem + static_cast<size_t>(rs.tb) * k * sizeof(AT), stream,
                        static_cast<const XT*>(x), static_cast<const AT*>(w), static_cast<const AT*>(bias), T, h, E, k,
                        score, normalize, static_cast<AT>(scale), rs, static_cast<AT*>(logits), topi,
                        static_cast<AT*>(gates));
@@ -715,14 +812,9 @@ extern "C" int rhp_route(const void* x, int x_dtype, const void* router_w, int r
     if (x_dtype == RHP_F32)
         return launch_route<float, float>(x, router_w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates,
                                           stream);
-    if (x_dtype == RHP_BF16) {
-        int not_taken = 0;
-        const int rc = launch_route_bf16(x, router_w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates,
-                                         stream, &not_taken);
-        if (!not_taken) return rc;
+    if (x_dtype == RHP_BF16)
         return launch_route<bf16, float>(x, router_w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates,
                                          stream);
-    }
     return fail(std::string("rhp_route: unsupported x dtype ") + dtype_name(x_dtype));
 }
 

@@ -66,6 +66,43 @@ def test_route_bit_exact(case):
     assert np.array_equal(gates.cpu().numpy().view(np.uint8), ref_gates.view(np.uint8)), "gate bits differ"
 
 
+# Edges of the matrix-core kernel: one token, a ragged last 16-token tile at both block sizes (16 and, from
+# 8192 bf16 tokens, 32), segment counts that are not a multiple of four, more segment quads than waves (the
+# sums continue over rounds), one expert, expert tiles over several rounds, and the LDS limits of its buffers.
+EDGE_CASES = [
+    ("one-token", 1, 4096, 8, 2, torch.bfloat16, "softmax", None, 0.02),
+    ("t8191", 8191, 256, 16, 2, torch.bfloat16, "softmax", None, 0.05),
+    ("t8197-wide", 8197, 512, 33, 4, torch.bfloat16, "sigmoid", "normal", 0.05),
+    ("t8192-wide-e250", 8192, 256, 250, 8, torch.bfloat16, "softmax", "zipf", 0.05),
+    ("five-segments", 77, 1280, 17, 3, torch.bfloat16, "softmax", None, 0.03),
+    ("sixteen-quads", 40, 16384, 24, 4, torch.bfloat16, "softmax", None, 0.01),
+    ("h8-e1", 50, 8, 1, 1, torch.bfloat16, "softmax", None, 0.3),
+    ("f32-h16384", 33, 16384, 12, 3, torch.float32, "sigmoid", "normal", 0.01),
+    ("f32-e400", 21, 256, 400, 16, torch.float32, "softmax", None, 0.05),
+    ("f64-e70", 35, 512, 70, 6, torch.float64, "sigmoid", "normal", 0.05),
+]
+
+
+@pytest.mark.parametrize("case", EDGE_CASES, ids=[c[0] for c in EDGE_CASES])
+def test_route_kernel_edges(case):
+    test_route_bit_exact(case)
+
+
+def test_route_ties_over_candidates():
+    # 130 experts in equal pairs two lanes' candidates apart: the lower id of each pair comes first.
+    T, h, E, k = 37, 256, 130, 8
+    x = seeded((T, h), 5, 1.0, torch.bfloat16)
+    w = seeded((E, h), 6, 0.05, torch.float32)
+    w[64:128] = w[0:64]
+    w[3] = w[2]
+    say("route ties over 130 experts")
+    logits, topi, gates = K.route(x.to(DEV), w.to(DEV), None, k, "softmax", True, 1.0)
+    ref_logits = R.router_logits(host_x(x), w.numpy(), "bf16")
+    ref_topi, ref_gates = R.topk(ref_logits, k)
+    assert np.array_equal(topi.cpu().numpy(), ref_topi)
+    assert np.array_equal(gates.cpu().numpy().view(np.uint8), ref_gates.view(np.uint8))
+
+
 def test_route_ties_and_nan():
     T, h, E, k = 64, 64, 16, 4
     x = seeded((T, h), 3, 1.0, torch.float32)
