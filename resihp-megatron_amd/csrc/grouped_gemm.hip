@@ -500,79 +500,257 @@ __global__ __launch_bounds__(64 * NW) void gg_bf16_kernel(Params p) {
     gg_bf16_tile<MODE, EPI, NW, REBASE, MAP>(p, t, lds);
 }
 
-// ------------------------------------------------------------------ generic kernel (any dtype)
+// ------------------------------------------------------------------ generic kernel (any dtype, any shape)
+//
+// float32 and float64 experts, and bfloat16 shapes the kernel above does not
+// take (h or f not a multiple of 64): a TM x TM output tile on four waves of
+// the matrix cores, in the operands' compute type (v_mfma_f32_16x16x4_f32,
+// bfloat16 widened to float32; v_mfma_f64_16x16x4_f64).  Every product is a
+// fused multiply-add of that type, as in a thread-per-output loop.
+//   Operands go through registers into a double-buffered LDS stage, KS of the
+// reduction (128 bytes a row) at a time, one barrier a step, the next step's
+// global loads in flight over the MFMAs.  A stage keeps its operand's memory
+// order, so no transposed copy or write is made:
+//     K contiguous:  [row][k], 144-byte rows (16 rows of a 16-byte read hit
+//                    distinct banks), a lane's four k in one read (f64: two);
+//     K slow:        [k][row], TM + 4 elements a k row (the four k groups of a
+//                    read are 16 words apart).
+// MFMA j of a 16-k block takes k = 4 q + j on the lanes of 16-lane group q, in
+// both operands: the order of k is free.  Elements past the reduction are
+// zeros in both operands.  Bound by the MFMAs and the LDS reads feeding them;
+// the forward and backward of 8 experts of 1024 by 2736 on 2000 float32 rows
+// (the whole layer): 39.3 ms with a thread per output reading operands from
+// memory, 1.26 ms on these tiles (80 of 153 TFLOP/s).
+constexpr int kGenericTile = 32;   // smallest extent of an output tile (activation columns, SwiGLU forward)
 
-// One thread per 4 outputs of a 32 x 32 tile, reading operands straight from
-// memory.  Used for float32 / float64 experts and for shapes the MFMA kernel
-// does not take (h or f not a multiple of 64); not a performance path.
-constexpr int kSimtTile = 32;
+template <class S> struct GenericK { static constexpr int KS = sizeof(typename Elem<S>::acc) == 8 ? 16 : 32; };
 
-template <class S, int MODE, int EPI>
-__global__ __launch_bounds__(256) void gg_simt_kernel(Params p) {
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
+template <class A> struct Mfma4;
+template <> struct Mfma4<float> {
+    using Acc = f32x4_t;
+    static __device__ __forceinline__ Acc run(float a, float b, Acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+    static __device__ __forceinline__ int row(int q, int e) { return 4 * q + e; }   // of accumulator element e
+};
+template <> struct Mfma4<double> {
+    using Acc = f64x4_t;
+    static __device__ __forceinline__ Acc run(double a, double b, Acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+    static __device__ __forceinline__ int row(int q, int e) { return q + 4 * e; }
+};
+
+// Four consecutive elements, as loaded and as compute values.
+template <class S> struct Quad {
+    S v[4];
+    __device__ __forceinline__ void zero() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = S{};
+    }
+    // n of them valid; VEC: all or none, through 8- or 16-byte loads.
+    template <bool VEC> __device__ __forceinline__ void load(const S* p, int n) {
+        if constexpr (VEC) {
+            if (n > 0) {
+                if constexpr (sizeof(S) == 2) *reinterpret_cast<uint2*>(v) = *reinterpret_cast<const uint2*>(p);
+                else
+#pragma unroll
+                    for (int i = 0; i < static_cast<int>(sizeof(S)) / 4; ++i)
+                        reinterpret_cast<uint4*>(v)[i] = reinterpret_cast<const uint4*>(p)[i];
+            } else {
+                zero();
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = i < n ? p[i] : S{};
+        }
+    }
+    __device__ __forceinline__ typename Elem<S>::acc get(int i) const { return Elem<S>::ld(v, i); }
+};
+
+// One operand of a tile: TM rows by KS of the reduction, staged in LDS.
+template <class S, int TM, bool KMAJ, bool VEC>
+struct GenericOperand {
     using A = typename Elem<S>::acc;
+    static constexpr int KS = GenericK<S>::KS, kUnits = TM * KS / 4 / 256;
+    static constexpr int kPitch = KMAJ ? 144 / static_cast<int>(sizeof(A)) : TM + 4;   // elements
+    static constexpr int kElems = (KMAJ ? TM : KS) * kPitch;
+    static_assert(kUnits >= 1, "every thread stages at least one quad");
+    const S* base[KMAJ ? kUnits : 1];   // KMAJ: the unit's row (null: zeros), else row 0's first column
+    int64_t ld;
+    int lim;                            // K slow: valid columns from base
+    Quad<S> r[kUnits];
+    __device__ __forceinline__ static int unit(int u) { return static_cast<int>(threadIdx.x) + 256 * u; }
+    __device__ __forceinline__ void load(int k0, int k_end) {
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            if constexpr (KMAJ) {
+                const int k = k0 + 4 * (unit(u) % (KS / 4));
+                if (base[u]) r[u].template load<VEC>(base[u] + k, k_end - k);
+                else r[u].zero();
+            } else {
+                const int k = k0 + unit(u) / (TM / 4), c = 4 * (unit(u) % (TM / 4));
+                r[u].template load<VEC>(base[0] + static_cast<int64_t>(k) * ld + c, k < k_end ? lim - c : 0);
+            }
+        }
+    }
+    __device__ __forceinline__ void stage(A* s) const {
+#pragma unroll
+        for (int u = 0; u < kUnits; ++u) {
+            A* d = KMAJ ? s + unit(u) / (KS / 4) * kPitch + 4 * (unit(u) % (KS / 4))
+                        : s + unit(u) / (TM / 4) * kPitch + 4 * (unit(u) % (TM / 4));
+            A v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = r[u].get(i);
+#pragma unroll
+            for (int i = 0; i < static_cast<int>(sizeof(A)) / 4; ++i)
+                reinterpret_cast<uint4*>(d)[i] = reinterpret_cast<const uint4*>(v)[i];
+        }
+    }
+    // The lane's four k of 16-k block kb for row `row`.
+    static __device__ __forceinline__ void frag(const A* s, int row, int q, int kb, A* f) {
+        if constexpr (KMAJ) {
+            const A* d = s + row * kPitch + 16 * kb + 4 * q;
+#pragma unroll
+            for (int i = 0; i < static_cast<int>(sizeof(A)) / 4; ++i)
+                reinterpret_cast<uint4*>(f)[i] = reinterpret_cast<const uint4*>(d)[i];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) f[j] = s[(16 * kb + 4 * q + j) * kPitch + row];
+        }
+    }
+};
+
+template <class S, int MODE, int EPI, int TM, bool VEC>
+__global__ __launch_bounds__(256) void gg_generic_kernel(Params p) {
+    using A = typename Elem<S>::acc;
+    using M = Mfma4<A>;
+    using YOp = GenericOperand<S, TM, MODE != kWgrad, VEC>;
+    using XOp = GenericOperand<S, TM, MODE == kFwd, VEC>;
+    constexpr int KS = GenericK<S>::KS, F = TM / 32;   // 16 x 16 fragments a wave and dimension (TM / 2 square)
+    constexpr int XC = EPI == kEpiSwigluFwd ? TM / 2 : TM;
+    __shared__ __align__(16) A ys[2][YOp::kElems];
+    __shared__ __align__(16) A xs[2][XOp::kElems];
     Tile t;
-    if (find_tile<MODE>(p, kSimtTile, kSimtTile, blockIdx.x, &t) != kTileOk) return;
+    if (find_tile<MODE>(p, XC, TM, blockIdx.x, &t) != kTileOk) return;
     const int g = t.g;
     const S* Ap = static_cast<const S*>(p.a[g]);
     const S* Bp = static_cast<const S*>(p.b[g]);
-    S* C = static_cast<S*>(p.c[g]);
-    const int y = threadIdx.x / 8;
-    if (y >= t.y_lim) return;
-    for (int e = 0; e < 4; ++e) {
-        const int xr = (threadIdx.x % 8) * 4 + e;
-        if (xr >= t.x_lim) continue;
-        const int col = t.x0 + xr;
-        A acc = A(0), acc_up = A(0);
-        if (MODE == kWgrad) {
-            for (int r = t.k_begin; r < t.k_end; ++r) {
-                const int64_t row = t.row0 + r;
-                acc += Elem<S>::ld(Ap, row * p.lda + t.y0 + y) * Elem<S>::ld(Bp, row * p.ldb + col);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+    const int wx = wave & 1, wy = wave >> 1;
+    // Column of row n of the X tile: SwiGLU forward tiles hold 16 gate rows, then the 16 up rows of the same
+    // columns, so a wave has both factors of an activation in neighbouring fragments.
+    auto x_col = [](int n) { return EPI == kEpiSwigluFwd ? (n / 32) * 16 + n % 16 : n; };
+
+    YOp yo;
+    XOp xo;
+    yo.ld = p.lda;
+    xo.ld = p.ldb;
+    if constexpr (MODE == kWgrad) {
+        yo.base[0] = Ap + t.row0 * p.lda + t.y0;
+        yo.lim = t.y_lim;
+        xo.base[0] = Bp + t.row0 * p.ldb + t.x0;
+        xo.lim = t.x_lim;
+    } else {
+#pragma unroll
+        for (int u = 0; u < YOp::kUnits; ++u) {
+            const int y = YOp::unit(u) / (KS / 4);
+            int64_t row = t.row0 + t.y0 + y;
+            if (y >= t.y_lim) {
+                row = -1;
+            } else if (p.a_idx) {   // row map: an index outside the buffer reads zeros
+                const int32_t s = p.a_idx[row];
+                row = s >= 0 && s < p.a_rows ? s : -1;
             }
-            Elem<S>::st(C, static_cast<int64_t>(t.y0 + y) * p.ldc + col, acc);
-            continue;
+            yo.base[u] = row >= 0 ? Ap + row * p.lda : nullptr;
         }
-        const int64_t row = t.row0 + t.y0 + y;
-        // Row maps: the token row read (a_idx) and the output row written (c_idx); -1 = none.
-        int64_t arow = row, crow = row;
-        if (p.a_idx) {
-            const int32_t s = p.a_idx[row];
-            arow = s >= 0 && s < p.a_rows ? s : -1;
-        }
-        if (p.c_idx) {
-            const int32_t s = p.c_idx[row];
-            crow = s >= 0 && s < p.c_rows ? s : -1;
-        }
-        for (int kk = 0; kk < p.K; ++kk) {
-            const A av = arow >= 0 ? Elem<S>::ld(Ap, arow * p.lda + kk) : A(0);
-            if (MODE == kFwd) {
-                acc += av * Elem<S>::ld(Bp, static_cast<int64_t>(col) * p.ldb + kk);
-                if (EPI == kEpiSwigluFwd) acc_up += av * Elem<S>::ld(Bp, static_cast<int64_t>(p.f + col) * p.ldb + kk);
-            } else {
-                acc += av * Elem<S>::ld(Bp, static_cast<int64_t>(kk) * p.ldb + col);
+        if constexpr (MODE == kFwd) {
+#pragma unroll
+            for (int u = 0; u < XOp::kUnits; ++u) {
+                const int n = XOp::unit(u) / (KS / 4), c = x_col(n);
+                const int64_t row = t.x0 + c + (EPI == kEpiSwigluFwd && n / 16 % 2 ? p.f : 0);
+                xo.base[u] = c < t.x_lim ? Bp + row * p.ldb : nullptr;
             }
-        }
-        if (EPI == kEpiStore) {
-            if (crow >= 0) Elem<S>::st(C, crow * p.ldc + col, acc);
-        } else if (EPI == kEpiStoreRouter) {
-            const A w = static_cast<A>(p.rw[static_cast<int64_t>(p.rw_e0 + g) * p.N + col]);
-            Elem<S>::st(C, row * p.ldc + col, acc + static_cast<A>(p.rdl[p.rperm[row]]) * w);
-        } else if (EPI == kEpiSwigluFwd) {
-            // the backward's factors [u silu'(g) | silu(g)] and the activation silu(g) u
-            Elem<S>::st(C, row * p.ldc + col, acc_up * dsilu_f(acc));
-            Elem<S>::st(C, row * p.ldc + p.f + col, silu_f(acc));
-            Elem<S>::st(static_cast<S*>(p.c2[g]), row * p.ldc2 + col, silu_f(acc) * acc_up);
-        } else if (EPI == kEpiGeluFwd) {
-            Elem<S>::st(C, row * p.ldc + col, acc);
-            Elem<S>::st(static_cast<S*>(p.c2[g]), row * p.ldc2 + col, gelu_f(acc));
-        } else if (EPI == kEpiSwigluBwd) {
-            const S* hp = static_cast<const S*>(p.aux[g]);
-            Elem<S>::st(C, row * p.ldc + col, acc * Elem<S>::ld(hp, row * p.ldaux + col));
-            Elem<S>::st(C, row * p.ldc + p.f + col, acc * Elem<S>::ld(hp, row * p.ldaux + p.f + col));
-        } else if (EPI == kEpiGeluBwd) {
-            const S* hp = static_cast<const S*>(p.aux[g]);
-            Elem<S>::st(C, row * p.ldc + col, acc * dgelu_f(Elem<S>::ld(hp, row * p.ldaux + col)));
+        } else {
+            xo.base[0] = Bp + t.x0;
+            xo.lim = t.x_lim;
         }
     }
+
+    typename M::Acc acc[F][F];
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = typename M::Acc{};
+    if (t.k_begin < t.k_end) {
+        yo.load(t.k_begin, t.k_end);
+        xo.load(t.k_begin, t.k_end);
+    }
+    int buf = 0;
+    for (int k0 = t.k_begin; k0 < t.k_end; k0 += KS, buf ^= 1) {
+        // The buffer written here was last read two steps ago, before the previous step's barrier.
+        yo.stage(ys[buf]);
+        xo.stage(xs[buf]);
+        if (k0 + KS < t.k_end) {
+            yo.load(k0 + KS, t.k_end);
+            xo.load(k0 + KS, t.k_end);
+        }
+        lds_barrier();   // the next step's global loads stay in flight
+#pragma unroll
+        for (int kb = 0; kb < KS / 16; ++kb) {
+            __align__(16) A yf[F][4], xf[F][4];
+#pragma unroll
+            for (int i = 0; i < F; ++i) YOp::frag(ys[buf], wy * (TM / 2) + 16 * i + r, q, kb, yf[i]);
+#pragma unroll
+            for (int j = 0; j < F; ++j) XOp::frag(xs[buf], wx * (TM / 2) + 16 * j + r, q, kb, xf[j]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int i = 0; i < F; ++i)
+#pragma unroll
+                    for (int j = 0; j < F; ++j) acc[i][j] = M::run(yf[i][k], xf[j][k], acc[i][j]);
+        }
+    }
+
+    S* C = static_cast<S*>(p.c[g]);
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int y = wy * (TM / 2) + 16 * i + M::row(q, e);
+            if (y >= t.y_lim) continue;
+            const int64_t row = MODE == kWgrad ? t.y0 + y : t.row0 + t.y0 + y;
+#pragma unroll
+            for (int j = 0; j < F; j += EPI == kEpiSwigluFwd ? 2 : 1) {
+                const int x = x_col(wx * (TM / 2) + 16 * j + r), col = t.x0 + x;
+                if (x >= t.x_lim) continue;
+                const A v = acc[i][j][e];
+                if (EPI == kEpiStore) {
+                    int64_t crow = row;
+                    if (MODE != kWgrad && p.c_idx) {   // row map: an index outside the buffer drops the row
+                        const int32_t s = p.c_idx[row];
+                        crow = s >= 0 && s < p.c_rows ? s : -1;
+                    }
+                    if (crow >= 0) Elem<S>::st(C, crow * p.ldc + col, v);
+                } else if (EPI == kEpiStoreRouter) {
+                    const A w = static_cast<A>(p.rw[static_cast<int64_t>(p.rw_e0 + g) * p.N + col]);
+                    Elem<S>::st(C, row * p.ldc + col, v + static_cast<A>(p.rdl[p.rperm[row]]) * w);
+                } else if (EPI == kEpiSwigluFwd) {
+                    // the backward's factors [u silu'(g) | silu(g)] and the activation silu(g) u
+                    const A up = acc[i][j + (EPI == kEpiSwigluFwd)][e], si = silu_f(v);
+                    Elem<S>::st(C, row * p.ldc + col, up * dsilu_f(v));
+                    Elem<S>::st(C, row * p.ldc + p.f + col, si);
+                    Elem<S>::st(static_cast<S*>(p.c2[g]), row * p.ldc2 + col, si * up);
+                } else if (EPI == kEpiGeluFwd) {
+                    Elem<S>::st(C, row * p.ldc + col, v);
+                    Elem<S>::st(static_cast<S*>(p.c2[g]), row * p.ldc2 + col, gelu_f(v));
+                } else if (EPI == kEpiSwigluBwd) {
+                    const S* hp = static_cast<const S*>(p.aux[g]);
+                    Elem<S>::st(C, row * p.ldc + col, v * Elem<S>::ld(hp, row * p.ldaux + col));
+                    Elem<S>::st(C, row * p.ldc + p.f + col, v * Elem<S>::ld(hp, row * p.ldaux + p.f + col));
+                } else if (EPI == kEpiGeluBwd) {
+                    const S* hp = static_cast<const S*>(p.aux[g]);
+                    Elem<S>::st(C, row * p.ldc + col, v * dgelu_f(Elem<S>::ld(hp, row * p.ldaux + col)));
+                }
+            }
+        }
 }
 
 // ------------------------------------------------------------------ host side
@@ -580,6 +758,7 @@ __global__ __launch_bounds__(256) void gg_simt_kernel(Params p) {
 struct Job {
     int mode, epi, dtype;
     bool mfma;
+    bool vec;         // generic kernel: quads of elements are aligned (run() finds out)
     int G;
     const int32_t* offsets;
     int rows_from_offsets;
@@ -617,9 +796,31 @@ int64_t mfma_blocks(const Params& p, int64_t rows_cap) {
     return row_grouped_blocks<MODE>(p, rows_cap, kTile, (p.N + x_per_tile<EPI>() - 1) / x_per_tile<EPI>());
 }
 
-template <int MODE>
-int64_t simt_blocks(const Params& p, int64_t rows_cap) {
-    return row_grouped_blocks<MODE>(p, rows_cap, kSimtTile, (p.N + kSimtTile - 1) / kSimtTile);
+template <int MODE, int EPI>
+int64_t generic_blocks(const Params& p, int64_t rows_cap, int tile) {
+    const int xc = EPI == kEpiSwigluFwd ? tile / 2 : tile;
+    return row_grouped_blocks<MODE>(p, rows_cap, tile, (p.N + xc - 1) / xc);
+}
+
+// Blocks of 128 x 128 tiles from which the generic kernel uses them; smaller products take 64 x 64 tiles, whose
+// four times as many blocks reach the CUs.
+constexpr int64_t kGenericWideBlocks = 512;
+
+template <class S, int MODE, int EPI>
+void launch_generic(const Job& j, const Params& p, hipStream_t s) {
+    if constexpr (sizeof(S) < 8) {
+        const int64_t nb = generic_blocks<MODE, EPI>(p, j.rows_cap, 128);
+        if (j.vec && nb >= kGenericWideBlocks) {
+            hipLaunchKernelGGL((gg_generic_kernel<S, MODE, EPI, 128, true>), dim3(static_cast<unsigned>(nb)), dim3(256), 0, s, p);
+            return;
+        }
+    }
+    const int64_t nb = generic_blocks<MODE, EPI>(p, j.rows_cap, 64);
+    if (!nb) return;
+    if (j.vec)
+        hipLaunchKernelGGL((gg_generic_kernel<S, MODE, EPI, 64, true>), dim3(static_cast<unsigned>(nb)), dim3(256), 0, s, p);
+    else
+        hipLaunchKernelGGL((gg_generic_kernel<S, MODE, EPI, 64, false>), dim3(static_cast<unsigned>(nb)), dim3(256), 0, s, p);
 }
 
 template <int MODE, int EPI>
@@ -650,14 +851,9 @@ void launch_one(const Job& j, const Params& p, hipStream_t s) {
         hipLaunchKernelGGL((gg_bf16_kernel<MODE, EPI, nw>), dim3(static_cast<unsigned>(nb)), dim3(64 * nw), 0, s, p);
         return;
     }
-    const unsigned nb = static_cast<unsigned>(simt_blocks<MODE>(p, j.rows_cap));
-    if (!nb) return;
-    if (j.dtype == RHP_BF16)
-        hipLaunchKernelGGL((gg_simt_kernel<bf16, MODE, EPI>), dim3(nb), dim3(256), 0, s, p);
-    else if (j.dtype == RHP_F32)
-        hipLaunchKernelGGL((gg_simt_kernel<float, MODE, EPI>), dim3(nb), dim3(256), 0, s, p);
-    else
-        hipLaunchKernelGGL((gg_simt_kernel<double, MODE, EPI>), dim3(nb), dim3(256), 0, s, p);
+    if (j.dtype == RHP_BF16) launch_generic<bf16, MODE, EPI>(j, p, s);
+    else if (j.dtype == RHP_F32) launch_generic<float, MODE, EPI>(j, p, s);
+    else launch_generic<double, MODE, EPI>(j, p, s);
 }
 
 void launch(const Job& j, const Params& p, hipStream_t s) {
@@ -674,13 +870,24 @@ void launch(const Job& j, const Params& p, hipStream_t s) {
     }
 }
 
+bool all_aligned(const void* const* ptrs, int G) {
+    if (!ptrs) return true;
+    for (int g = 0; g < G; ++g)
+        if (!aligned16(ptrs[g])) return false;
+    return true;
+}
+
 // Runs a job in launches of at most kMaxG groups.
 int run(const Job& job, const char* what, hipStream_t s) {
     Job j = job;
     j.cus_per_xcd = cus_per_xcd();
+    // Quad loads need operands aligned to 16 bytes and rows of whole quads (a quad then is valid or past
+    // its row as a whole); other operands are read element by element.
+    j.vec = j.lda % 4 == 0 && j.ldb % 4 == 0 && j.K % 4 == 0 && j.N % 4 == 0 && j.Mo % 4 == 0 &&
+            all_aligned(j.a, j.G) && all_aligned(j.b, j.G);
     {
         // Every launch's grid (an upper bound of its tiles, plus a K split's extra round) fits in 31 bits.
-        const int64_t tr = j.mfma ? kTile : kSimtTile, tx = j.mfma ? 128 : kSimtTile;
+        const int64_t tr = j.mfma ? kTile : kGenericTile, tx = j.mfma ? 128 : kGenericTile;
         const int64_t g = std::min(j.G, kMaxG), xt = (j.N + tx - 1) / tx;
         const int64_t bound = j.mode == kWgrad ? wgrad_blocks(g, xt * ((j.Mo + tr - 1) / tr))
                                                : ((j.rows_cap + tr - 1) / tr + 1) * g * xt + kXcds * kSplitMaxCus;
@@ -733,13 +940,6 @@ int run(const Job& job, const char* what, hipStream_t s) {
         if (int rc = check_launch(what)) return rc;
     }
     return 0;
-}
-
-bool all_aligned(const void* const* ptrs, int G) {
-    if (!ptrs) return true;
-    for (int g = 0; g < G; ++g)
-        if (!aligned16(ptrs[g])) return false;
-    return true;
 }
 
 bool all_set(const void* const* ptrs, int G) {

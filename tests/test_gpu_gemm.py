@@ -112,6 +112,50 @@ def test_grouped_expert_gemms(case, act):
         assert rel_err(c64(dw1[g]), dh_g[r0:r1].t() @ xs) <= bar, ("dw1", g)
 
 
+# The generic kernel's edges: reductions and columns that end inside a stage, a quad and a 16-wide fragment
+# (sizes that are and are not multiples of four: quad and element loads), row tiles of 1, 63, 64, 65 and 129
+# rows, empty groups, and products large enough for its 128 x 128 tiles.
+GENERIC_CASES = [
+    ("f32-elements", torch.float32, 72, 50, [1, 63, 0, 64, 65, 129]),
+    ("f32-quads", torch.float32, 136, 100, [1, 63, 0, 64, 65, 129]),
+    ("f32-wide", torch.float32, 1032, 1028, [257, 1, 0, 640, 127, 129, 300, 90]),
+    ("f64-elements", torch.float64, 40, 27, [1, 63, 0, 64, 65, 129]),
+    ("f64-quads", torch.float64, 136, 100, [70, 1, 0, 129]),
+    ("bf16-elements", torch.bfloat16, 72, 51, [1, 63, 0, 64, 65, 129]),
+    ("bf16-wide", torch.bfloat16, 1032, 1028, [257, 1, 0, 640, 127, 129, 300, 90]),
+]
+
+
+@pytest.mark.parametrize("act", ["swiglu", "gelu"])
+@pytest.mark.parametrize("case", GENERIC_CASES, ids=[c[0] for c in GENERIC_CASES])
+def test_generic_kernel_edges(case, act):
+    test_grouped_expert_gemms(case, act)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float64], ids=str)
+def test_generic_kernel_unaligned_operands(dt):
+    """Operands one element past a 16-byte boundary (element loads) give the aligned operands' product."""
+    h, f, M = 64, 96, 77
+    off = torch.tensor([0, M], dtype=torch.int32, device=DEV)
+
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, dtype=dt, device=DEV)
+        buf[1:] = t.reshape(-1).to(DEV)
+        return buf[1:].view(t.shape)
+
+    x, w1, w2 = seeded((M, h), 1, 1.0, dt), seeded((2 * f, h), 2, 0.05, dt), seeded((h, f), 3, 0.05, dt)
+    say(f"unaligned generic operands {dt}")
+    outs = []
+    for put in (lambda t: t.to(DEV), shifted):
+        hpre, a, y = (torch.empty(M, n, dtype=dt, device=DEV) for n in (2 * f, f, h))
+        K.expert_fc1_fwd([put(x)], off, False, M, [put(w1)], f, "swiglu", [hpre], [a])
+        K.expert_fc2_fwd([a], off, False, M, [put(w2)], [y])
+        outs.append((hpre, a, y))
+    torch.cuda.synchronize()
+    for p, q in zip(*outs):
+        assert torch.equal(p, q)
+
+
 @pytest.mark.parametrize("T", [200, 513, 2048])
 def test_per_group_buffers_shared_expert_mode(T):
     """rows_from_offsets = 0: each group reads and writes its own buffer from row 0 (shared experts).
