@@ -92,16 +92,12 @@ def lib() -> ctypes.CDLL:
 
 def call(name: str, *args) -> None:
     """Calls an entry point and turns a nonzero status into RuntimeError."""
-    L = lib()
-    rc = getattr(L, name)(*args)
+    rc = getattr(_lib or lib(), name)(*args)
     if rc != 0:
-        msg = L.rhp_last_error().decode(errors="replace")
+        msg = lib().rhp_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed: {msg}")
 
 
 def ptr_array(ptrs) -> ctypes.Array:
     """Host array of device pointers (``const void* const*``)."""
-    arr = (ctypes.c_void_p * max(1, len(ptrs)))()
-    for i, p in enumerate(ptrs):
-        arr[i] = p
-    return arr
+    return (ctypes.c_void_p * max(1, len(ptrs)))(*ptrs)

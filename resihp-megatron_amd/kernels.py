@@ -33,6 +33,11 @@ def set_timer(timer) -> None:
 
 def _call(name: str, dev: torch.device, *args) -> None:
     """Calls entry point ``name`` with ``args`` and the current stream of ``dev``."""
+    if _timer is None and torch.cuda.current_device() == dev.index:
+        # The usual case, without the objects that the device guard and the stream wrapper make (about
+        # 6 us a call, of some twenty calls a layer pass).
+        C.call(name, *args, torch._C._cuda_getCurrentRawStream(dev.index))
+        return
     stream = torch.cuda.current_stream(dev)
     with torch.cuda.device(dev):
         if _timer is not None:
@@ -53,9 +58,62 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def _need_cuda(*ts: torch.Tensor | None) -> torch.device:
-    dev = None
+class Group:
+    """The tensors of a list of groups, found to be of one 2-D shape, dtype and HIP device and contiguous,
+    with their pointer array: what a call checks and converts per tensor, done once for the calls that one
+    forward or backward makes with them.  Not kept beyond it."""
+
+    __slots__ = ("ts", "arr", "dtype", "shape", "device")
+
+    def __init__(self, ts):
+        self.ts = ts
+        self.arr = C.ptr_array([t.data_ptr() for t in ts])
+        self.dtype, self.shape, self.device = ts[0].dtype, ts[0].shape, ts[0].device
+
+    def __len__(self) -> int:
+        return len(self.ts)
+
+    def __getitem__(self, i):
+        return self.ts[i]
+
+
+def group(ts):
+    """``ts`` as a Group where its tensors are alike (see there), else as it is, for the calls to judge."""
+    ts = list(ts)
+    if not ts:
+        return ts
+    t0 = ts[0]
+    dt, shape, dev = t0.dtype, t0.shape, t0.get_device()
+    if dev < 0 or len(shape) != 2:
+        return ts
     for t in ts:
+        if t.dtype is not dt or t.get_device() != dev or not t.is_contiguous() or t.shape != shape:
+            return ts
+    return Group(ts)
+
+
+def _distinct(ts):
+    """The tensors of a list that differ from the one before: one, where every group shares a buffer."""
+    out, last = [], None
+    for t in ts:
+        if t is not last:
+            out.append(t)
+            last = t
+    return out
+
+
+def _need_cuda(*ts) -> torch.device:
+    """The HIP device of tensors, lists of tensors, Groups and Nones."""
+    flat = []
+    for t in ts:
+        if isinstance(t, Group):
+            flat.append(t.ts[0])   # the others are alike
+        elif isinstance(t, (list, tuple)):
+            flat.extend(_distinct(t))
+        else:
+            flat.append(t)
+    dev = None
+    for t in flat:
         if t is None:
             continue
         if not t.is_cuda:
@@ -363,14 +421,26 @@ def gather_rows(src: torch.Tensor, idx: torch.Tensor, out: torch.Tensor | None =
 
 
 def _arr(ts) -> object:
+    if isinstance(ts, Group):
+        return ts.arr
+    if len(ts) > 1 and all(t is ts[0] for t in ts):
+        return C.ptr_array([ts[0].data_ptr()] * len(ts))
     return C.ptr_array([t.data_ptr() for t in ts])
 
 
 def _check_groups(what: str, ts: list[torch.Tensor], G: int, dtype: torch.dtype, cols: int,
                   rows: int | None = None, exact_shape: tuple[int, int] | None = None) -> None:
     """Every group tensor must have the kernel's dtype and shape; the kernels cannot see either."""
-    _expect(len(ts) == G, f"{what}: expected {G} tensors, got {len(ts)}")
-    for i, t in enumerate(ts):
+    if len(ts) != G:
+        raise KernelArgumentError(f"{what}: expected {G} tensors, got {len(ts)}")
+    last = None
+    for i, t in enumerate(ts.ts[:1] if isinstance(ts, Group) else ts):
+        if t is last:
+            continue
+        last, shape = t, t.shape
+        if (t.dtype is dtype and len(shape) == 2 and shape[1] == cols
+                and (exact_shape is None or shape[0] == exact_shape[0]) and (rows is None or shape[0] >= rows)):
+            continue
         _expect(t.dtype == dtype, f"{what}[{i}] has dtype {t.dtype}, expected {dtype}")
         _expect(t.dim() == 2, f"{what}[{i}] must be 2-D")
         _expect(exact_shape is None or tuple(t.shape) == exact_shape,
@@ -419,13 +489,15 @@ def split_workspace(dev: torch.device, stream: torch.cuda.Stream | None = None) 
     fails resets them.  Under HIP graph capture a workspace is never allocated: make one call outside
     the capture on the same stream first, or the call raises.
     """
-    idx = torch.device(dev).index if torch.device(dev).index is not None else torch.cuda.current_device()
-    stream = stream if stream is not None else torch.cuda.current_stream(idx)
-    key = (idx, stream.cuda_stream)
+    idx = dev.index if isinstance(dev, torch.device) else torch.device(dev).index
+    if idx is None:
+        idx = torch.cuda.current_device()
+    key = (idx, torch._C._cuda_getCurrentRawStream(idx) if stream is None else stream.cuda_stream)
     ws = _split_ws_cache.get(key)
     if ws is not None:
         _split_ws_cache.move_to_end(key)
         return ws
+    stream = stream if stream is not None else torch.cuda.current_stream(idx)
     if torch.cuda.is_current_stream_capturing():
         raise KernelArgumentError("the expert GEMMs' K-split workspace of this stream is not allocated: "
                                   "call them once on this stream before capturing a graph")
@@ -462,7 +534,7 @@ def _split_call(name: str, dev: torch.device, split: bool, *args) -> None:
 def expert_fc1_fwd(xs: list[torch.Tensor], offsets: torch.Tensor, rows_from_offsets: bool, rows_cap: int,
                    w1: list[torch.Tensor], f: int, act: str, hpre: list[torch.Tensor],
                    act_out: list[torch.Tensor], split: bool = True) -> None:
-    dev = _need_cuda(offsets, *xs, *w1, *hpre, *act_out)
+    dev = _need_cuda(offsets, xs, w1, hpre, act_out)
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     rows = _shared_rows(rows_from_offsets, rows_cap)
@@ -477,7 +549,7 @@ def expert_fc1_fwd(xs: list[torch.Tensor], offsets: torch.Tensor, rows_from_offs
 
 def expert_fc2_fwd(acts: list[torch.Tensor], offsets: torch.Tensor, rows_from_offsets: bool, rows_cap: int,
                    w2: list[torch.Tensor], ys: list[torch.Tensor], split: bool = True) -> None:
-    dev = _need_cuda(offsets, *acts, *w2, *ys)
+    dev = _need_cuda(offsets, acts, w2, ys)
     G, dt, (h, f) = len(w2), w2[0].dtype, tuple(w2[0].shape)
     rows = _shared_rows(rows_from_offsets, rows_cap)
     _check_offsets(offsets, G)
@@ -494,7 +566,7 @@ def expert_fc2_bwd(dys: list[torch.Tensor], acts: list[torch.Tensor], hpres: lis
     """Input-gradient product into ``dhpre`` and weight gradient into ``dw2``; either may be None (not
     both), so the two independent products can run on two streams.  ``w2`` gives the shapes either way."""
     _expect(dhpre is not None or dw2 is not None, "expert_fc2_bwd: nothing to compute")
-    dev = _need_cuda(offsets, *dys, *acts, *hpres, *w2, *(dhpre or []), *(dw2 or []))
+    dev = _need_cuda(offsets, dys, acts, hpres, w2, dhpre, dw2)
     G, dt, (h, f) = len(w2), w2[0].dtype, tuple(w2[0].shape)
     F1 = 2 * f if act == "swiglu" else f
     rows = _shared_rows(rows_from_offsets, rows_cap)
@@ -518,7 +590,7 @@ def expert_fc1_bwd(dhpre: list[torch.Tensor], xs: list[torch.Tensor], offsets: t
                    dxs: list[torch.Tensor] | None, dw1: list[torch.Tensor] | None, split: bool = True) -> None:
     """Input gradient into ``dxs`` and weight gradient into ``dw1``; either may be None (not both)."""
     _expect(bool(dxs) or dw1 is not None, "expert_fc1_bwd: nothing to compute")
-    dev = _need_cuda(offsets, *dhpre, *xs, *w1, *(dxs or []), *(dw1 or []))
+    dev = _need_cuda(offsets, dhpre, xs, w1, dxs, dw1)
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     rows = _shared_rows(rows_from_offsets, rows_cap)
@@ -544,7 +616,7 @@ def expert_fc1_fwd_gather(src: torch.Tensor, src_idx: torch.Tensor, offsets: tor
                           w1: list[torch.Tensor], f: int, act: str, hpre: torch.Tensor, act_out: torch.Tensor,
                           split: bool = True) -> None:
     """expert_fc1_fwd on rows gathered from ``src``: grouped row r is ``src[src_idx[r]]`` (no copy)."""
-    dev = _need_cuda(offsets, src, src_idx, *w1, hpre, act_out)
+    dev = _need_cuda(offsets, src, src_idx, w1, hpre, act_out)
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     _check_offsets(offsets, G)
@@ -560,7 +632,7 @@ def expert_fc1_fwd_gather(src: torch.Tensor, src_idx: torch.Tensor, offsets: tor
 def expert_fc2_fwd_scatter(act_in: torch.Tensor, offsets: torch.Tensor, rows_cap: int, w2: list[torch.Tensor],
                            y: torch.Tensor, y_idx: torch.Tensor, split: bool = True) -> None:
     """expert_fc2_fwd writing grouped row r to ``y[y_idx[r]]`` (no copy)."""
-    dev = _need_cuda(offsets, act_in, y, y_idx, *w2)
+    dev = _need_cuda(offsets, act_in, y, y_idx, w2)
     G, dt, (h, f) = len(w2), w2[0].dtype, tuple(w2[0].shape)
     _check_offsets(offsets, G)
     _check_map("y_idx", y_idx, rows_cap)
@@ -575,7 +647,7 @@ def expert_fc2_dgrad_gather(dy: torch.Tensor, dy_idx: torch.Tensor, offsets: tor
                             w2: list[torch.Tensor], act: str, hpre: torch.Tensor, dhpre: torch.Tensor,
                             split: bool = True) -> None:
     """The input-gradient product of expert_fc2_bwd on output-gradient rows ``dy[dy_idx[r]]`` (no copy)."""
-    dev = _need_cuda(offsets, dy, dy_idx, hpre, dhpre, *w2)
+    dev = _need_cuda(offsets, dy, dy_idx, hpre, dhpre, w2)
     G, dt, (h, f) = len(w2), w2[0].dtype, tuple(w2[0].shape)
     F1 = 2 * f if act == "swiglu" else f
     _check_offsets(offsets, G)
@@ -591,7 +663,7 @@ def expert_fc2_dgrad_gather(dy: torch.Tensor, dy_idx: torch.Tensor, offsets: tor
 def expert_fc1_dgrad_scatter(dhpre: torch.Tensor, offsets: torch.Tensor, rows_cap: int, w1: list[torch.Tensor],
                              f: int, act: str, dx: torch.Tensor, dx_idx: torch.Tensor, split: bool = True) -> None:
     """The input-gradient product of expert_fc1_bwd writing grouped row r to ``dx[dx_idx[r]]`` (no copy)."""
-    dev = _need_cuda(offsets, dhpre, dx, dx_idx, *w1)
+    dev = _need_cuda(offsets, dhpre, dx, dx_idx, w1)
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     _check_offsets(offsets, G)
@@ -608,7 +680,7 @@ def expert_fc1_dgrad_router(dhpre: list[torch.Tensor], offsets: torch.Tensor, ro
                             dxs: list[torch.Tensor], split: bool = True) -> None:
     """fc1's input gradient with the router term added per row: ``dxs[r] = dhpre[r] @ w1 + dl[perm[r]] *
     router_w[e0 + g]`` (then token_bwd runs without ``dl``).  Every expert of the layer must be local."""
-    dev = _need_cuda(offsets, router_w, perm, dl, *dhpre, *w1, *dxs)
+    dev = _need_cuda(offsets, router_w, perm, dl, dhpre, w1, dxs)
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     _check_offsets(offsets, G)

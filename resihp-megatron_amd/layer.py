@@ -89,7 +89,7 @@ def expert_backward(dys, acts, hpres, offsets, rows_from_offsets: bool, rows_cap
     The weight gradients go to the side stream when the products run concurrently (CONCURRENT_BACKWARD);
     the current stream waits for them before returning, so every output is ordered on it as usual.
     ``router`` = (router_w, e0, perm, dl) folds the router term into fc1's input gradient."""
-    fc1s, fc2s = list(fc1s), list(fc2s)
+    fc1s, fc2s, dw1, dw2 = K.group(fc1s), K.group(fc2s), K.group(dw1), K.group(dw2)
 
     def fc1_dgrad():
         if router is None:
@@ -199,13 +199,13 @@ class _MoELayerFn(torch.autograd.Function):
         e0, e1 = meta.window
         G = e1 - e0
         S = meta.num_shared
-        fc1s, fc2s = list(weights[:G]), list(weights[G:2 * G])
+        fc1s, fc2s = K.group(weights[:G]), K.group(weights[G:2 * G])
         sfc1s, sfc2s = list(weights[2 * G:2 * G + S]), list(weights[2 * G + S:2 * G + 2 * S])
         T, h = x.shape
         k, f = meta.top_k, meta.ffn
         fs = meta.shared_ffn or f
         shared_off = shared_h = shared_a = shared_y = None
-        K.need_device(x, router_w, *weights)
+        K.need_device(x, router_w, fc1s, fc2s, sfc1s, sfc2s)
         main = torch.cuda.current_stream(x.device)
         # Shared experts need only x: concurrently with the routing and the routed experts on a side
         # stream where the products run concurrently, else after them.
@@ -222,7 +222,7 @@ class _MoELayerFn(torch.autograd.Function):
                 K.expert_fc1_fwd([x] * S, shared_off, False, T, sfc1s, fs, meta.act, shared_h, shared_a)
                 K.expert_fc2_fwd(shared_a, shared_off, False, T, sfc2s, shared_y)
         # fp8 experts (never with shared experts): the weight casts start now, on the side stream.
-        wcast = _fp8_weight_casts(fp8, fc1s, fc2s, main) if fp8 is not None else None
+        wcast = _fp8_weight_casts(fp8, weights[:G], weights[G:2 * G], main) if fp8 is not None else None
         logits, topi, gates = K.route(x, router_w, bias, k, meta.score, meta.normalize, meta.gate_scale)
         plan = K.dispatch(topi, meta.num_experts, e0, e1, meta.n_src)
         # The reference materialises counts on the host here too (moe.py:210-211);
@@ -252,7 +252,7 @@ class _MoELayerFn(torch.autograd.Function):
         ctx.fp8 = (fp8, q8)
         ctx.dims = (T, h, P, G, S)
         ctx.save_for_backward(x, router_w, logits, topi, gates, plan.perm, plan.offsets, plan.pair_row, xp, hpre,
-                              act, y, *fc1s, *fc2s, *sfc1s, *sfc2s)
+                              act, y, *weights)
         ctx.shared = (shared_off, shared_h, shared_a)
         ctx.mark_non_differentiable(plan.counts)
         return out, plan.counts
@@ -349,7 +349,7 @@ class _ExpertChunksFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, act, f, rows, recv_counts, recv, *weights):
         G = len(weights) // 2
-        fc1s, fc2s = list(weights[:G]), list(weights[G:])
+        fc1s, fc2s = K.group(weights[:G]), K.group(weights[G:])
         plan = K.recv_plan(recv_counts, rows)
         P, h = plan.rows, recv.shape[1]
         if recv.shape[0] != P:
@@ -369,7 +369,7 @@ class _ExpertChunksFn(torch.autograd.Function):
             K.expert_fc2_fwd_scatter(a, plan.offsets, P, fc2s, y, plan.sort_row)
             main.wait_stream(side)
         ctx.act, ctx.f, ctx.P = act, f, P
-        ctx.save_for_backward(plan.offsets, plan.sort_row, xs, hpre, a, *fc1s, *fc2s)
+        ctx.save_for_backward(plan.offsets, plan.sort_row, xs, hpre, a, *weights)
         return y
 
     @staticmethod
@@ -382,7 +382,9 @@ class _ExpertChunksFn(torch.autograd.Function):
         dw2 = [torch.empty_like(w) for w in fc2s]
         drecv = None
         need_x = ctx.needs_input_grad[4]
+        grads = (*dw1, *dw2)
         if P > 0:
+            fc1s, fc2s, dw1, dw2 = K.group(fc1s), K.group(fc2s), K.group(dw1), K.group(dw2)
             dy_recv = dy_recv.contiguous()
             h = xs.shape[1]
             dys = torch.empty_like(xs)          # expert-major output gradients, for the fc2 weight gradient
@@ -415,7 +417,7 @@ class _ExpertChunksFn(torch.autograd.Function):
             for w in (*dw1, *dw2):
                 w.zero_()
             drecv = torch.zeros_like(xs)
-        return (None, None, None, None, drecv, *dw1, *dw2)
+        return (None, None, None, None, drecv, *grads)
 
 
 def expert_chunks(recv: torch.Tensor, recv_counts: torch.Tensor, fc1s: list[torch.Tensor],
