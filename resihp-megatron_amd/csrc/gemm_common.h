@@ -48,6 +48,7 @@ struct Params {
     int32_t* split_cnt;       // [8 * cu_per_xcd] arrival counters, zero between launches
     int split_cap;
     int cu_per_xcd;
+    int split_piece_k;        // reduction length a piece keeps at least
     int split_kstep;          // the kernel's K step: pieces start and end on multiples of it
     // Quantising epilogues (fp8 kernels): the activation (forward) or the
     // pre-activation gradient (backward) leaves as fp8 codes instead of bf16,
@@ -137,9 +138,16 @@ constexpr int kXcds = 8;
 // A split pays only where a tile's reduction is long: each piece publishes
 // a 256 KB partial tile behind an L2-wide release, and the last one reads all
 // of them back.  Measured at K = 1408-4096 the split lost up to 8 %, at
-// K = 14336 and 28672 it gained 4 % and 2 %.
+// K = 14336 and 28672 it gained 4 % and 2 %.  Where groups hold few rows the
+// partial tiles are only the 16-row fragments that hold any, and the launch
+// streams weights: its time is its rounds of tiles, and a last round of a few
+// tiles costs a whole one unless they are split (8 experts of 4096 by 14336, 8
+// tokens, 806 fc1 tiles on 256 CUs).
 constexpr int kSplitMinK = 8192;        // reduction length a tile needs to be split at all
 constexpr int kSplitMinPieceK = 1024;   // reduction length a split piece keeps at least
+constexpr int kSplitFewRows = 64;       // average rows a group up to which the lengths below hold instead
+constexpr int kSplitFewMinK = 2048;
+constexpr int kSplitFewPieceK = 512;
 
 // K-split workspace: 8 XCDs x up to kSplitMaxCus pieces of one fp32 tile each,
 // then one arrival counter per piece slot.
@@ -256,9 +264,9 @@ __device__ __forceinline__ int find_tile(const Params& p, int xt_cols, int yt_ro
         const uint32_t q = total / kXcds, r = total % kXcds;
         const uint32_t n = q + (x < r ? 1u : 0u), start = x * q + (x < r ? x : r);
         const uint32_t F = n / C * C, rx = n - F;
-        uint32_t s = rx && p.K >= kSplitMinK ? C / rx : 1u;
+        uint32_t s = rx ? C / rx : 1u;   // (the host sets split_cap only for reductions that may be split)
         s = min(s, static_cast<uint32_t>(p.split_cap));
-        s = min(s, static_cast<uint32_t>(p.K / kSplitMinPieceK));
+        s = min(s, static_cast<uint32_t>(p.K / p.split_piece_k));
         if (j < F || s < 2) {
             if (j >= n) return kTileDone;
             L = start + j;
@@ -387,7 +395,7 @@ constexpr int kFragY = kWaveY / 32;                        // Y fragments per wa
 //     X 16 i + 4 (lane >> 4) + e, Y 16 j + (lane & 15) in v[i][j][e].
 template <int WY>
 struct Acc32 {
-    static constexpr int FY = WY / 32, kVec = 16 * FY;
+    static constexpr int FY = WY / 32, kVec = 16 * FY, kXW = 128;
     f32x16_t v[4][FY];
     __device__ __forceinline__ void zero() {
 #pragma unroll
@@ -402,23 +410,20 @@ struct Acc32 {
     }
     static __device__ __forceinline__ int x(int n, int lane) { return 32 * (n / (4 * FY)) + 8 * (n % 4) + 4 * (lane >> 5); }
     static __device__ __forceinline__ int y(int n, int lane) { return 32 * ((n / 4) % FY) + (lane & 31); }
+    static __device__ __forceinline__ int y_first(int n) { return 32 * ((n / 4) % FY); }
 };
-template <int WY>
+//     WX = 64: the wave's share is 64 X wide (the tiles of at most 128 rows).
+template <int WY, int WX = 128>
 struct Acc16 {
-    static constexpr int FY = WY / 16, kVec = 8 * FY;
-    f32x4_t v[8][FY];
-    __device__ __forceinline__ void zero() {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int j = 0; j < FY; ++j) v[i][j] = f32x4_t{};
-    }
+    static constexpr int FY = WY / 16, FX = WX / 16, kVec = FX * FY, kXW = WX;
+    f32x4_t v[FX][FY];
     __device__ __forceinline__ float4 get(int n) const {
         const f32x4_t& a = v[n / FY][n % FY];
         return make_float4(a[0], a[1], a[2], a[3]);
     }
     static __device__ __forceinline__ int x(int n, int lane) { return 16 * (n / FY) + 4 * (lane >> 4); }
     static __device__ __forceinline__ int y(int n, int lane) { return 16 * (n % FY) + (lane & 15); }
+    static __device__ __forceinline__ int y_first(int n) { return 16 * (n % FY); }
 };
 
 // Chunk swizzle of MN-major tiles: chunk c of k row k sits at c ^ mn_swz(k).
@@ -1042,11 +1047,12 @@ __device__ __forceinline__ void epilogue_pass(const Params& p, const Tile& t, fl
     if constexpr (EPI == kEpiStoreRouter) dst_rows = __float_as_int(router_scale_half<NT>(p, t, HALF * kEpRows));
     lds_barrier();
     if ((wy * wy_rows) / kEpRows == HALF) {
-        float* wave_ep = ep + (wy * wy_rows - HALF * kEpRows) * kEpPitchF + wx * 128;
+        float* wave_ep = ep + (wy * wy_rows - HALF * kEpRows) * kEpPitchF + wx * Acc::kXW;
         if (split.pieces) {
             // The sum of the pieces, in piece order.
 #pragma unroll
             for (int n = 0; n < Acc::kVec; ++n) {
+                if (wy * wy_rows + Acc::y_first(n) >= t.y_lim) continue;   // no piece holds it, no store wants it
                 const float4* src = split.first + n * NT + threadIdx.x;
                 float4 v = src[0];
                 for (int pc = 1; pc < split.pieces; ++pc) {
@@ -1104,12 +1110,13 @@ template <int MODE, int EPI, int NT, int WY, int QF = -1, bool MAP = false, clas
 __device__ __forceinline__ void epilogue(const Params& p, const Tile& t, uint8_t* lds, const Acc& acc, int wx, int wy,
                                          int lane, float mul = 1.0f, SplitSum split = SplitSum{nullptr, 0, 0}) {
     static_assert(WY <= kEpRows && kEpRows % WY == 0, "a wave's rows lie in one half");
-    static_assert(NT * Acc::kVec * 4 == kTile * kTile, "the waves' accumulators cover the tile");
+    constexpr bool kShort = NT * Acc::kVec * 4 == kTile * kEpRows;   // a tile of at most 128 rows: its first half
+    static_assert(kShort || NT * Acc::kVec * 4 == kTile * kTile, "the waves' accumulators cover the tile");
     float* ep = reinterpret_cast<float*>(lds);
     QuantAcc qa{1.0f, 0.0f};
     if constexpr (QF >= 0) qa.scale = history_scale(p.q_hist, p.q_L, fp8_max(QF), p.q_margin);
     epilogue_pass<0, MODE, EPI, NT, QF, MAP>(p, t, ep, acc, wx, wy, WY, lane, mul, split, qa);
-    epilogue_pass<1, MODE, EPI, NT, QF, MAP>(p, t, ep, acc, wx, wy, WY, lane, mul, split, qa);
+    if constexpr (!kShort) epilogue_pass<1, MODE, EPI, NT, QF, MAP>(p, t, ep, acc, wx, wy, WY, lane, mul, split, qa);
     if constexpr (QF >= 0) {
         // Wave maximum, then one atomic per wave; non-negative floats order like
         // their bits, and a maximum not above the value read (possibly stale,
@@ -1125,19 +1132,21 @@ __device__ __forceinline__ void epilogue(const Params& p, const Tile& t, uint8_t
 }
 
 // A piece of a K-split tile: every piece stores its fp32 accumulators (laid
-// out thread-major, so each store instruction of a wave is contiguous), makes
+// out thread-major, so each store instruction of a wave is contiguous; not the
+// fragments past the tile's valid rows, wy_row0 being the wave's first), makes
 // them visible device-wide and counts itself in.  The piece that arrives last
 // returns true: its epilogue then stages the sum of all pieces, read from
 // memory in piece order (the same bits whichever piece is last), instead of
 // its own accumulators.  It resets the counter for the next launch.  No block
 // ever waits for another.
 template <int NT, class Acc>
-__device__ __forceinline__ bool split_arrive(const Params& p, const Tile& t, const Acc& acc, uint8_t* lds) {
-    static_assert(NT * Acc::kVec * 4 == kTile * kTile, "a piece holds a whole tile");
+__device__ __forceinline__ bool split_arrive(const Params& p, const Tile& t, const Acc& acc, uint8_t* lds, int wy_row0) {
+    static_assert(NT * Acc::kVec * 4 <= kTile * kTile, "a piece holds a whole tile, or a tile of at most 128 rows");
     const int tid = threadIdx.x;
-    float4* mine = reinterpret_cast<float4*>(p.split_part) + static_cast<size_t>(t.slot + t.piece * t.stride) * (NT * Acc::kVec);
+    float4* mine = reinterpret_cast<float4*>(p.split_part) + static_cast<size_t>(t.slot + t.piece * t.stride) * (kTile * kTile / 4);
 #pragma unroll
-    for (int n = 0; n < Acc::kVec; ++n) mine[n * NT + tid] = acc.get(n);
+    for (int n = 0; n < Acc::kVec; ++n)
+        if (wy_row0 + Acc::y_first(n) < t.y_lim) mine[n * NT + tid] = acc.get(n);
     // Each wave waits for its own stores; after the barrier one thread makes
     // the whole block's stores visible device-wide and counts the piece in.
     // (An agent-scope fence writes back the XCD's L2; one per piece, not one

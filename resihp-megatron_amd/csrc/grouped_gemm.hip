@@ -484,11 +484,180 @@ __device__ __forceinline__ void gg_bf16_tile(const Params& p, Tile t, uint8_t* l
 #pragma unroll
         for (int j = 0; j < FY; ++j) out.v[i][j] = acc[i][j];
     if (MODE != kWgrad && t.pieces > 1) {
-        if (!split_arrive<64 * NW>(p, t, out, lds)) return;
+        if (!split_arrive<64 * NW>(p, t, out, lds, wy * WY)) return;
         epilogue<MODE, EPI, 64 * NW, WY, -1, MAP>(p, t, lds, out, wx, wy, lane, 1.0f, split_sum_of(p, t));
         return;
     }
     epilogue<MODE, EPI, 64 * NW, WY, -1, MAP>(p, t, lds, out, wx, wy, lane);
+}
+
+// The tile of a group of at most 128 rows (row-grouped products): the same ring
+// of operand slots, with four waves of 64 X by 128 Y rows, so every SIMD works on
+// the rows there are.  (The 128 x 128 split above leaves the two waves of the
+// lower rows idle: a K step takes the time of a full tile.)  A Y slot holds
+// 128 rows, half the loads; each block of 32 MFMAs carries 12 fragment reads
+// (forward; 16 with the input gradients' half-reads) and 8 or 4 loads, one
+// memory instruction after each of its first MFMAs, loads spread evenly.
+//   Bound by the weights' HBM traffic; with the K split of few-row launches
+// (kSplitFewRows), 8 tokens by 8 experts of 4096 by 14336: fc1 forward 374 ->
+// 310 us (4.5 -> 5.4 TB/s), fc2 forward 211 -> 149 (4.0 -> 5.7); 64 tokens by 64
+// experts of 2048 by 1408, top 6: 155 -> 125 and 71 -> 60 us.
+template <int MODE, int EPI, bool MAP>
+__device__ __forceinline__ void gg_bf16_short_tile(const Params& p, Tile t, uint8_t* lds) {
+    constexpr int NW = 4, FX = 4, FY = 8;
+    constexpr int kXLoads = kT64Bytes / 1024 / NW, kYLoads = kXLoads / 2;   // per wave and operand tile
+    constexpr bool kXK = MODE == kFwd;
+    t.g = __builtin_amdgcn_readfirstlane(t.g);
+    t.x0 = __builtin_amdgcn_readfirstlane(t.x0);
+    t.x_lim = __builtin_amdgcn_readfirstlane(t.x_lim);
+    t.y0 = __builtin_amdgcn_readfirstlane(t.y0);
+    t.y_lim = __builtin_amdgcn_readfirstlane(t.y_lim);
+    t.row0 = __builtin_amdgcn_readfirstlane(static_cast<int>(t.row0));
+    t.k_begin = __builtin_amdgcn_readfirstlane(t.k_begin);
+    t.k_end = __builtin_amdgcn_readfirstlane(t.k_end);
+    t.piece = __builtin_amdgcn_readfirstlane(t.piece);
+    t.pieces = __builtin_amdgcn_readfirstlane(t.pieces);
+    t.slot = __builtin_amdgcn_readfirstlane(t.slot);
+    t.stride = __builtin_amdgcn_readfirstlane(t.stride);
+    const int g = t.g;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    const uint16_t* A = static_cast<const uint16_t*>(p.a[g]);
+    const uint16_t* B = static_cast<const uint16_t*>(p.b[g]);
+    const uint32_t ldb = static_cast<uint32_t>(p.ldb), lda = static_cast<uint32_t>(p.lda);
+    Rsrc rx, ry;
+    Dma64Map<NW> mx, my;
+    const int y_last = t.y_lim - 1;
+    if (MAP && p.a_idx != nullptr) {   // gathered token rows, as in gg_bf16_tile
+        ry = make_dma_rsrc(A, p.a_rows * p.lda * 2);
+        const int32_t* ix = p.a_idx + t.row0 + t.y0;
+        const uint32_t n_rows = static_cast<uint32_t>(p.a_rows);
+        d64_kmaj(my, lda, 0, FY, [&](int r) {
+            const uint32_t src = static_cast<uint32_t>(ix[r < t.y_lim ? r : y_last]);
+            return src < n_rows ? src : n_rows;
+        });
+    } else {
+        ry = make_dma_rsrc(A + (t.row0 + t.y0) * p.lda, static_cast<int64_t>(t.y_lim) * p.lda * 2);
+        d64_kmaj(my, lda, 0, FY, [&](int r) { return r < t.y_lim ? r : y_last; });
+    }
+    if (MODE == kFwd) {
+        rx = make_dma_rsrc(B, static_cast<int64_t>(EPI == kEpiSwigluFwd ? 2 * p.f : p.N) * p.ldb * 2);
+        d64_kmaj(mx, ldb, wave * 64, FX, [&](int r) {
+            if (EPI == kEpiSwigluFwd) {   // [gate 64 | up 64] for each half of 128 activation columns
+                const int half = r >> 7, qq = r & 127;
+                int col = t.x0 + half * 64 + (qq & 63);
+                col = col < p.f ? col : 0;
+                return qq < 64 ? col : p.f + col;
+            }
+            const int n = t.x0 + r;
+            return n < p.N ? n : 0;
+        });
+    } else {
+        rx = make_dma_rsrc(B, static_cast<int64_t>(p.K) * p.ldb * 2);
+        d64_mnmaj(mx, ldb, t.x0, t.x_lim, wave * 64, FX);
+    }
+    const int nk = (t.k_end - t.k_begin + kK64 - 1) / kK64;
+    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+    auto issue_x = [&](int step, int slot, int j0, int j1) {
+        const uint32_t k0 = static_cast<uint32_t>(t.k_begin + step * kK64);
+        const bool live = step < nk;
+        const uint32_t base = lds0 + slot * kT64Bytes + wave * 1024;
+#pragma unroll
+        for (int j = j0; j < j1; ++j) {
+            const uint32_t at = base + j * NW * 1024;
+            if (kXK) dma16(rx, mx.vo[j], live ? k0 * 2u : kPastView, at);
+            else dma16(rx, mx.vo[j] + (live ? k0 * ldb * 2u : 0u), live ? 0u : kPastView, at);
+        }
+    };
+    auto issue_y = [&](int step, int slot, int j0, int j1) {
+        const uint32_t k0 = static_cast<uint32_t>(t.k_begin + step * kK64);
+        const uint32_t base = lds0 + slot * kT64Bytes + wave * 1024;
+#pragma unroll
+        for (int j = j0; j < j1; ++j) dma16(ry, my.vo[j], step < nk ? k0 * 2u : kPastView, base + j * NW * 1024);
+    };
+    auto wait_lds = [](auto n_c) {   // vmcnt(n loads of this wave) lgkmcnt(0)
+        constexpr int n = decltype(n_c)::value;
+        __builtin_amdgcn_s_waitcnt(0x0070 | (n & 15) | ((n >> 4) << 14));
+    };
+    auto barrier = [] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    f32x4_t acc[FX][FY];
+#pragma unroll
+    for (int i = 0; i < FX; ++i)
+#pragma unroll
+        for (int j = 0; j < FY; ++j) acc[i][j] = f32x4_t{};
+    typedef bf16x8_t YSet[FY];
+    bf16x8_t xf[2][FX];
+    auto kfrag = [](const uint8_t* tile, uint32_t fr, int b) {
+        return *reinterpret_cast<const bf16x8_t*>(tile + (fr ^ static_cast<uint32_t>(b << 6)));
+    };
+    auto read_x = [&](int set, uint32_t sx, int b, int i) {
+        xf[set][i] = kXK ? kfrag(lds + sx, mx.fr[i], b) : frag_mn32(lds + sx, mx.fr[i], b);
+    };
+    auto read_y = [&](YSet& y, uint32_t sy, int b, int j) { y[j] = kfrag(lds + sy, my.fr[j], b); };
+    auto block = [&](const YSet& yc, YSet& yn, int xc, int xn, uint32_t sx, uint32_t sy, int b, auto load, auto n_c) {
+        constexpr int n = decltype(n_c)::value, kOps = FY + FX + n;
+        static_assert(kOps <= FX * FY, "memory instructions fit between the MFMAs");
+#pragma unroll
+        for (int m = 0; m < FX * FY; ++m) {
+            mfma16<NW>(acc[m / FY][m % FY], xf[xc][m / FY], yc[m % FY]);
+            if (m < kOps) {
+                const int l = m * n / kOps;              // loads issued before
+                if ((m + 1) * n / kOps > l) load(l);
+                else if (m - l < FY) read_y(yn, sy, b, m - l);
+                else read_x(xn, sx, b, m - l - FY);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    using XPending = std::integral_constant<int, kXLoads>;
+    using YPending = std::integral_constant<int, kYLoads>;
+    using Prolog = std::integral_constant<int, kXLoads + kYLoads>;
+    YSet ya, yb;
+    if (nk > 0) {
+        issue_x(0, 0, 0, kXLoads);
+        issue_y(0, 1, 0, kYLoads);
+        issue_x(1, 2, 0, kXLoads);
+        issue_y(1, 3, 0, kYLoads);
+        wait_lds(Prolog{});   // step 0 complete
+        barrier();
+#pragma unroll
+        for (int j = 0; j < FY; ++j) read_y(ya, kT64Bytes, 0, j);
+#pragma unroll
+        for (int i = 0; i < FX; ++i) read_x(0, 0, 0, i);
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0), as in gg_bf16_tile
+        int sx = 0, sy = 1, nx = 2, ny = 3, fx = 4;
+        for (int kt = 0; kt < nk; ++kt) {
+            mfma_srcc_ready<NW>();
+            block(ya, yb, 0, 1, sx * kT64Bytes, sy * kT64Bytes, 1, [&](int l) { issue_x(kt + 2, fx, l, l + 1); }, XPending{});
+            wait_lds(XPending{});   // steps up to kt + 1 complete, X of step kt + 2 in flight
+            barrier();
+            block(yb, ya, 1, 0, nx * kT64Bytes, ny * kT64Bytes, 0, [&](int l) { issue_y(kt + 2, sx, l, l + 1); }, YPending{});
+            const int x2 = fx, y2 = sx;
+            fx = sy;
+            sx = nx;
+            sy = ny;
+            nx = x2;
+            ny = y2;
+        }
+        wait_loads_all();   // the tiles past the last step
+    }
+    mfma_drain<NW>();
+    Acc16<128, 64> out;
+#pragma unroll
+    for (int i = 0; i < FX; ++i)
+#pragma unroll
+        for (int j = 0; j < FY; ++j) out.v[i][j] = acc[i][j];
+    if (t.pieces > 1) {
+        if (!split_arrive<64 * NW>(p, t, out, lds, 0)) return;
+        epilogue<MODE, EPI, 64 * NW, 128, -1, MAP>(p, t, lds, out, wave, 0, lane, 1.0f, split_sum_of(p, t));
+        return;
+    }
+    epilogue<MODE, EPI, 64 * NW, 128, -1, MAP>(p, t, lds, out, wave, 0, lane);
 }
 
 // One block per tile (hardware block b runs on XCD b % 8).
@@ -497,6 +666,15 @@ __global__ __launch_bounds__(64 * NW) void gg_bf16_kernel(Params p) {
     __shared__ __align__(1024) uint8_t lds[kLdsSlotsBytes];
     Tile t;
     if (find_tile<MODE>(p, x_per_tile<EPI>(), kTile, blockIdx.x, &t) != kTileOk) return;
+    if constexpr (MODE != kWgrad) {
+        // Only groups that have no full tile: they are bound by the weights' way to the CUs.  At the end of a
+        // larger group (or beside other full tiles) the GPU is at its power limit, where the idle waves cost
+        // nothing and the short tile gains nothing: a 1500-token Mixtral forward ran 3 % slower with it.
+        if (__builtin_amdgcn_readfirstlane(t.y_lim + t.y0) <= kTile / 2) {
+            gg_bf16_short_tile<MODE, EPI, MAP>(p, t, lds);
+            return;
+        }
+    }
     gg_bf16_tile<MODE, EPI, NW, REBASE, MAP>(p, t, lds);
 }
 
@@ -926,12 +1104,14 @@ int run(const Job& job, const char* what, hipStream_t s) {
         p.rw_e0 = j.rw_e0 + g0;
         // Only reductions long enough to be split get the split (and its larger
         // grid: the extra, mostly empty blocks cost about 1 % of a short product).
-        if (j.split_ws && j.mfma && j.mode != kWgrad && j.K >= kSplitMinK) {
+        const bool few = j.rows_cap <= static_cast<int64_t>(kSplitFewRows) * (j.rows_from_offsets ? gn : 1);
+        if (j.split_ws && j.mfma && j.mode != kWgrad && j.K >= (few ? kSplitFewMinK : kSplitMinK)) {
             const int C = std::min(kSplitMaxCus, j.cus_per_xcd);
             if (C > 1) {
                 p.split_part = static_cast<float*>(j.split_ws);
                 p.split_cnt = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(j.split_ws) + kSplitPartBytes);
                 p.split_cap = kSplitCap;
+                p.split_piece_k = few ? kSplitFewPieceK : kSplitMinPieceK;
                 p.cu_per_xcd = C;
                 p.split_kstep = 64;
             }

@@ -112,6 +112,23 @@ def test_grouped_expert_gemms(case, act):
         assert rel_err(c64(dw1[g]), dh_g[r0:r1].t() @ xs) <= bar, ("dw1", g)
 
 
+# Groups of few rows on the bf16 kernel: tiles of at most 128 rows (1, a fragment and its neighbours, 127, 128;
+# 129 takes a full tile), and their reduction split along K (at most 64 rows a group on average, from 2048),
+# also beside one group of several full tiles.
+FEW_ROW_CASES = [
+    ("short-tiles", torch.bfloat16, 320, 192, [1, 15, 16, 17, 127, 128, 129, 0]),
+    ("short-split", torch.bfloat16, 2048, 2112, [1, 0, 16, 17, 64, 128, 33, 129]),
+    ("short-split-ragged-k", torch.bfloat16, 2112, 2496, [40]),
+    ("hot-group-split", torch.bfloat16, 2048, 2048, [600, 1] + [0] * 14),
+]
+
+
+@pytest.mark.parametrize("act", ["swiglu", "gelu"])
+@pytest.mark.parametrize("case", FEW_ROW_CASES, ids=[c[0] for c in FEW_ROW_CASES])
+def test_few_rows_per_group(case, act):
+    test_grouped_expert_gemms(case, act)
+
+
 # The generic kernel's edges: reductions and columns that end inside a stage, a quad and a 16-wide fragment
 # (sizes that are and are not multiples of four: quad and element loads), row tiles of 1, 63, 64, 65 and 129
 # rows, empty groups, and products large enough for its 128 x 128 tiles.
