@@ -33,10 +33,16 @@ namespace {
 
 constexpr int kAdamMax = 64;        // tensors per launch
 constexpr int kAdamThreads = 256;
-// 8-element groups per thread: 64 bytes of each of the four arrays in flight
-// per thread (4 groups of bfloat16, 2 of float32, 1 of float64).
-template <class S> constexpr int adam_groups() { return 8 / static_cast<int>(sizeof(S)); }
-template <class S> constexpr int64_t adam_block_elems() { return int64_t(kAdamThreads) * adam_groups<S>() * 8; }
+// Elements per thread.  One 8-element group of each of the four arrays, all
+// loads and stores non-temporal (nothing is read twice): the step is bound by
+// HBM, and small blocks that come and go keep its reads and writes mixed.
+// 1.41 G bfloat16 parameters (14 bytes each, 256 threads a block): 4 groups a
+// thread with ordinary accesses 3664 us, 5.39 TB/s; non-temporal 3479; 2
+// groups 3487; 1 group 3305, 5.97 TB/s (ordinary accesses 3573).  Cutting a
+// quarter of the instructions (shorter exact square root and divisions)
+// changed none of these by more than 2 %, so the plain forms stay.
+constexpr int kAdamElems = 8;
+constexpr int64_t kAdamBlockElems = int64_t(kAdamThreads) * kAdamElems;
 
 struct AdamTensors {
     void* p[kAdamMax];
@@ -108,7 +114,7 @@ __device__ __forceinline__ void adam_one(const AdamScalars<typename AdamElem<S>:
 // Two bfloat16 elements at once, operation for operation as adam_one: each
 // operation's two results are rounded by one v_cvt_pk_bf16_f32 (the rounding
 // AdamElem<bf16>::r applies to each value alone, so the bits are the same)
-// instead of one conversion per value; the step is bound by VALU issue.
+// instead of one conversion per value.
 __device__ __forceinline__ void round2(float& x, float& y) {
     const uint32_t b = pack_bf16x2(x, y);
     x = __uint_as_float(b << 16);
@@ -146,15 +152,16 @@ __device__ __forceinline__ void adam_two_bf16(const AdamScalars<float>& sc, floa
 
 // Raw 16-byte groups of 8 elements.
 template <class S> struct Group8 {
+    typedef uint32_t Word __attribute__((ext_vector_type(4)));
     static constexpr int kWords = static_cast<int>(sizeof(S)) * 8 / 16;
-    uint4 w[kWords];
+    Word w[kWords];
     __device__ __forceinline__ void load(const S* p) {
 #pragma unroll
-        for (int i = 0; i < kWords; ++i) w[i] = reinterpret_cast<const uint4*>(p)[i];
+        for (int i = 0; i < kWords; ++i) w[i] = __builtin_nontemporal_load(reinterpret_cast<const Word*>(p) + i);
     }
     __device__ __forceinline__ void store(S* p) const {
 #pragma unroll
-        for (int i = 0; i < kWords; ++i) reinterpret_cast<uint4*>(p)[i] = w[i];
+        for (int i = 0; i < kWords; ++i) __builtin_nontemporal_store(w[i], reinterpret_cast<Word*>(p) + i);
     }
     __device__ __forceinline__ S& at(int e) { return reinterpret_cast<S*>(w)[e]; }
 };
@@ -169,79 +176,70 @@ template <> __device__ __forceinline__ float from_t<float>(float x) { return x; 
 template <> __device__ __forceinline__ bf16 from_t<bf16>(float x) { return bf16{AdamElem<bf16>::bits(x)}; }
 
 // Block b updates elements [B * (b - block0[t]), +B) of tensor t, B =
-// adam_block_elems<S>(): each thread kG groups of 8 consecutive elements, all
-// loads of a thread issued before the first update.
+// kAdamBlockElems: each thread 8 consecutive elements, all loads issued before
+// the first update.
 template <class S>
 __global__ __launch_bounds__(kAdamThreads) void adam_kernel(AdamTensors ts, AdamScalars<typename AdamElem<S>::T> sc) {
     using T = typename AdamElem<S>::T;
-    constexpr int kG = adam_groups<S>();
-    int t = 0;
-    while (t + 1 < ts.count && blockIdx.x >= ts.block0[t + 1]) ++t;
+    // The block's tensor: one candidate per lane (a scalar load per tensor in turn took longer than the update).
+    static_assert(kAdamMax <= 64, "one tensor per lane");
+    const int lane = static_cast<int>(threadIdx.x & 63);
+    const bool past = lane + 1 < ts.count && blockIdx.x >= ts.block0[min(lane + 1, kAdamMax)];
+    const int t = __builtin_amdgcn_readfirstlane(static_cast<int>(__popcll(__ballot(past))));
     const int64_t n = ts.n[t];
     S* P = static_cast<S*>(ts.p[t]);
     const S* G = static_cast<const S*>(ts.g[t]);
     S* M = static_cast<S*>(ts.m[t]);
     S* V = static_cast<S*>(ts.v[t]);
-    const int64_t base = static_cast<int64_t>(blockIdx.x - ts.block0[t]) * adam_block_elems<S>();
-    const int64_t full = n / 8 * 8;   // elements in whole 8-element groups
-    Group8<S> gp[kG], gg[kG], gm[kG], gv[kG];
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x - ts.block0[t]) * kAdamBlockElems + threadIdx.x * kAdamElems;
+    if (e0 < n / 8 * 8) {   // a whole 8-element group
+        Group8<S> gp, gg, gm, gv;
+        gp.load(P + e0);
+        gm.load(M + e0);
+        gv.load(V + e0);
+        if (G) gg.load(G + e0);
+        if constexpr (std::is_same<S, bf16>::value) {
 #pragma unroll
-    for (int q = 0; q < kG; ++q) {
-        const int64_t e0 = base + (static_cast<int64_t>(q) * kAdamThreads + threadIdx.x) * 8;
-        if (e0 < full) {
-            gp[q].load(P + e0);
-            gm[q].load(M + e0);
-            gv[q].load(V + e0);
-            if (G) gg[q].load(G + e0);
-        }
-    }
+            for (int e = 0; e < 8; e += 2) {
+                float p[2], g[2], m[2], v[2];
 #pragma unroll
-    for (int q = 0; q < kG; ++q) {
-        const int64_t e0 = base + (static_cast<int64_t>(q) * kAdamThreads + threadIdx.x) * 8;
-        if (e0 < full) {
-            if constexpr (std::is_same<S, bf16>::value) {
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    float p[2], g[2], m[2], v[2];
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        p[i] = to_t<S>(gp[q].at(e + i));
-                        m[i] = to_t<S>(gm[q].at(e + i));
-                        v[i] = to_t<S>(gv[q].at(e + i));
-                        g[i] = G ? to_t<S>(gg[q].at(e + i)) : 0.0f;
-                    }
-                    adam_two_bf16(sc, p, g, m, v);
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        gp[q].at(e + i) = from_t<S>(p[i]);
-                        gm[q].at(e + i) = from_t<S>(m[i]);
-                        gv[q].at(e + i) = from_t<S>(v[i]);
-                    }
+                for (int i = 0; i < 2; ++i) {
+                    p[i] = to_t<S>(gp.at(e + i));
+                    m[i] = to_t<S>(gm.at(e + i));
+                    v[i] = to_t<S>(gv.at(e + i));
+                    g[i] = G ? to_t<S>(gg.at(e + i)) : 0.0f;
                 }
-            } else {
+                adam_two_bf16(sc, p, g, m, v);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    T p = to_t<S>(gp[q].at(e)), m = to_t<S>(gm[q].at(e)), v = to_t<S>(gv[q].at(e));
-                    const T g = G ? to_t<S>(gg[q].at(e)) : T(0);
-                    adam_one<S>(sc, p, g, m, v);
-                    gp[q].at(e) = from_t<S>(p);
-                    gm[q].at(e) = from_t<S>(m);
-                    gv[q].at(e) = from_t<S>(v);
+                for (int i = 0; i < 2; ++i) {
+                    gp.at(e + i) = from_t<S>(p[i]);
+                    gm.at(e + i) = from_t<S>(m[i]);
+                    gv.at(e + i) = from_t<S>(v[i]);
                 }
             }
-            gp[q].store(P + e0);
-            gm[q].store(M + e0);
-            gv[q].store(V + e0);
-        } else if (e0 < n) {
-            // The last, partial group of the tensor: element by element.
-            for (int64_t i = e0; i < n; ++i) {
-                T p = AdamElem<S>::ld(P, i), m = AdamElem<S>::ld(M, i), v = AdamElem<S>::ld(V, i);
-                const T g = G ? AdamElem<S>::ld(G, i) : T(0);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                T p = to_t<S>(gp.at(e)), m = to_t<S>(gm.at(e)), v = to_t<S>(gv.at(e));
+                const T g = G ? to_t<S>(gg.at(e)) : T(0);
                 adam_one<S>(sc, p, g, m, v);
-                AdamElem<S>::st(P, i, p);
-                AdamElem<S>::st(M, i, m);
-                AdamElem<S>::st(V, i, v);
+                gp.at(e) = from_t<S>(p);
+                gm.at(e) = from_t<S>(m);
+                gv.at(e) = from_t<S>(v);
             }
+        }
+        gp.store(P + e0);
+        gm.store(M + e0);
+        gv.store(V + e0);
+    } else if (e0 < n) {
+        // The last, partial group of the tensor: element by element.
+        for (int64_t i = e0; i < n; ++i) {
+            T p = AdamElem<S>::ld(P, i), m = AdamElem<S>::ld(M, i), v = AdamElem<S>::ld(V, i);
+            const T g = G ? AdamElem<S>::ld(G, i) : T(0);
+            adam_one<S>(sc, p, g, m, v);
+            AdamElem<S>::st(P, i, p);
+            AdamElem<S>::st(M, i, m);
+            AdamElem<S>::st(V, i, v);
         }
     }
 }
@@ -260,7 +258,7 @@ int launch_adam(int count, void* const* params, const void* const* grads, void* 
             ts.v[i] = v[t0 + i];
             ts.n[i] = numel[t0 + i];
             ts.block0[i] = static_cast<uint32_t>(blocks);
-            blocks += static_cast<uint64_t>((numel[t0 + i] + adam_block_elems<S>() - 1) / adam_block_elems<S>());
+            blocks += static_cast<uint64_t>((numel[t0 + i] + kAdamBlockElems - 1) / kAdamBlockElems);
         }
         ts.block0[ts.count] = static_cast<uint32_t>(blocks);
         RHP_REQUIRE(blocks < (uint64_t(1) << 31), "rhp_adam_step: too many elements in one launch");

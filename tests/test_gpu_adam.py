@@ -59,6 +59,33 @@ def test_fused_adam_matches_oracle_bitwise(dtype, wd):
                 assert np.array_equal(_bits(_np(t)), _bits(a)), (dtype, wd, step, SIZES[i], what)
 
 
+@pytest.mark.parametrize("kind", ["ordinary", "any-bits", "eps0", "beta2-1", "beta1-small"])
+def test_bf16_step_over_all_magnitudes(kind):
+    """bfloat16 tensors over every second-moment value and wide numerators, and over random bit patterns with
+    infinities, NaN, zeros, subnormals and negative second moments."""
+    n = 1 << 18
+    g = torch.Generator().manual_seed(77)
+    bits = lambda: torch.randint(-32768, 32768, (n,), generator=g, dtype=torch.int32).to(torch.int16)  # noqa: E731
+    if kind == "any-bits":
+        p, gr, m, v = (bits().view(torch.bfloat16) for _ in range(4))
+    else:
+        p, gr, m = ((torch.randn(n, generator=g) * 10.0 ** (6 * torch.randn(n, generator=g))).to(torch.bfloat16)
+                    for _ in range(3))
+        v = torch.arange(n, dtype=torch.int32).remainder(0x7f80).to(torch.int16).view(torch.bfloat16)
+    betas = {"beta2-1": (0.9, 1.0), "beta1-small": (0.3, 0.99)}.get(kind, (0.9, 0.999))
+    eps = 0.0 if kind == "eps0" else 1e-8
+    host = [_np(p), _np(m), _np(v)]
+    dev = [t.to(DEV) for t in (p, m, v)]
+    say(f"adam bf16 {kind}")
+    with np.errstate(all="ignore"):
+        for step in (1, 2, 1000):
+            K.adam_step([dev[0]], [gr.to(DEV)], [dev[1]], [dev[2]], 1e-3, betas, eps, 0.1, step)
+            adam_c.adam_step(host[0], _np(gr), host[1], host[2], 1e-3, betas, eps, 0.1, step)
+            torch.cuda.synchronize()
+            for t, a, what in zip(dev, host, ("param", "exp_avg", "exp_avg_sq")):
+                assert np.array_equal(_bits(_np(t)), _bits(a)), (kind, step, what)
+
+
 def test_fused_adam_many_tensors_one_call():
     """More tensors than one launch takes (64): the call splits them; every one is updated."""
     g = torch.Generator().manual_seed(5)
