@@ -687,15 +687,16 @@ __global__ __launch_bounds__(64 * NW) void gg_bf16_kernel(Params p) {
 // fused multiply-add of that type, as in a thread-per-output loop.
 //   Operands go through registers into a double-buffered LDS stage, KS of the
 // reduction (128 bytes a row) at a time, one barrier a step, the next step's
-// global loads in flight over the MFMAs.  A stage keeps its operand's memory
-// order, so no transposed copy or write is made:
+// global loads in flight over the MFMAs.  MFMA j of a 16-k block takes
+// k = 4 j + q on the lanes of 16-lane group q, and adds its four products one
+// after the other: every output is one ascending chain over k, as a loop over k
+// in a thread gives it, bit for bit.  Stages:
 //     K contiguous:  [row][k], 144-byte rows (16 rows of a 16-byte read hit
-//                    distinct banks), a lane's four k in one read (f64: two);
-//     K slow:        [k][row], TM + 4 elements a k row (the four k groups of a
-//                    read are 16 words apart).
-// MFMA j of a 16-k block takes k = 4 q + j on the lanes of 16-lane group q, in
-// both operands: the order of k is free.  Elements past the reduction are
-// zeros in both operands.  Bound by the MFMAs and the LDS reads feeding them;
+//                    distinct banks), each block of 16 k transposed as 4 x 4 on
+//                    its way in, so a lane's four k come in one read (f64: two);
+//     K slow:        [k][row] as in memory, TM + 16 elements a k row (the four
+//                    k of a read are 16 words apart).
+// Elements past the reduction are zeros in both operands.  Bound by the MFMAs and the LDS reads feeding them;
 // the forward and backward of 8 experts of 1024 by 2736 on 2000 float32 rows
 // (the whole layer): 39.3 ms with a thread per output reading operands from
 // memory, 1.26 ms on these tiles (80 of 153 TFLOP/s).
@@ -748,7 +749,7 @@ template <class S, int TM, bool KMAJ, bool VEC>
 struct GenericOperand {
     using A = typename Elem<S>::acc;
     static constexpr int KS = GenericK<S>::KS, kUnits = TM * KS / 4 / 256;
-    static constexpr int kPitch = KMAJ ? 144 / static_cast<int>(sizeof(A)) : TM + 4;   // elements
+    static constexpr int kPitch = KMAJ ? 144 / static_cast<int>(sizeof(A)) : TM + 16;   // elements
     static constexpr int kElems = (KMAJ ? TM : KS) * kPitch;
     static_assert(kUnits >= 1, "every thread stages at least one quad");
     const S* base[KMAJ ? kUnits : 1];   // KMAJ: the unit's row (null: zeros), else row 0's first column
@@ -772,17 +773,23 @@ struct GenericOperand {
     __device__ __forceinline__ void stage(A* s) const {
 #pragma unroll
         for (int u = 0; u < kUnits; ++u) {
-            A* d = KMAJ ? s + unit(u) / (KS / 4) * kPitch + 4 * (unit(u) % (KS / 4))
-                        : s + unit(u) / (TM / 4) * kPitch + 4 * (unit(u) % (TM / 4));
             A v[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = r[u].get(i);
+            if constexpr (KMAJ) {
+                const int c = unit(u) % (KS / 4);   // k 4 c + i goes to place 4 i + c mod 4 of its block
+                A* d = s + unit(u) / (KS / 4) * kPitch + 16 * (c / 4) + c % 4;
 #pragma unroll
-            for (int i = 0; i < static_cast<int>(sizeof(A)) / 4; ++i)
-                reinterpret_cast<uint4*>(d)[i] = reinterpret_cast<const uint4*>(v)[i];
+                for (int i = 0; i < 4; ++i) d[4 * i] = v[i];
+            } else {
+                A* d = s + unit(u) / (TM / 4) * kPitch + 4 * (unit(u) % (TM / 4));
+#pragma unroll
+                for (int i = 0; i < static_cast<int>(sizeof(A)) / 4; ++i)
+                    reinterpret_cast<uint4*>(d)[i] = reinterpret_cast<const uint4*>(v)[i];
+            }
         }
     }
-    // The lane's four k of 16-k block kb for row `row`.
+    // The lane's four k (4 j + q) of 16-k block kb for row `row`.
     static __device__ __forceinline__ void frag(const A* s, int row, int q, int kb, A* f) {
         if constexpr (KMAJ) {
             const A* d = s + row * kPitch + 16 * kb + 4 * q;
@@ -791,7 +798,7 @@ struct GenericOperand {
                 reinterpret_cast<uint4*>(f)[i] = reinterpret_cast<const uint4*>(d)[i];
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) f[j] = s[(16 * kb + 4 * q + j) * kPitch + row];
+            for (int j = 0; j < 4; ++j) f[j] = s[(16 * kb + 4 * j + q) * kPitch + row];
         }
     }
 };

@@ -149,6 +149,34 @@ def test_generic_kernel_edges(case, act):
     test_grouped_expert_gemms(case, act)
 
 
+@pytest.mark.parametrize("h,f,M", [(50, 51, 65), (132, 100, 130)])
+def test_generic_kernel_adds_in_order(h, f, M):
+    """Every float32 output is one ascending chain of fused multiply-adds over its reduction, in all three
+    products.  Values of 8 bits: a product is exact in float64, and so is its sum with a float32 (no more than
+    53 bits from the sum's first to the product's last), so rounding that sum is the fused multiply-add."""
+    bf = lambda shape, seed, std: seeded(shape, seed, std, torch.bfloat16).float()  # noqa: E731
+    dy, a, w2 = bf((M, h), 1, 1.0), bf((M, f), 2, 1.0), bf((h, f), 3, 1.0)
+    off = torch.tensor([0, M], dtype=torch.int32, device=DEV)
+    d = lambda t: t.to(DEV)  # noqa: E731
+    y, dw = torch.empty(M, h, device=DEV), torch.empty(h, f, device=DEV)
+    dxs, dg = torch.empty(M, f, device=DEV), torch.empty(M, h, device=DEV)
+    say(f"generic order h={h} f={f} M={M}")
+    K.expert_fc2_fwd([d(a)], off, False, M, [d(w2)], [y])
+    K.expert_fc2_bwd([d(dy)], [d(a)], [d(dg)], off, False, M, [d(w2)], "gelu", None, [dw])
+    K.expert_fc1_bwd([d(dy)], [d(a)], off, False, M, [d(w2)], h, "gelu", [dxs], None)
+    torch.cuda.synchronize()
+
+    def chain(p, q):   # sum over r of p[:, r] q[r, :]
+        acc = torch.zeros(p.shape[0], q.shape[1])
+        for r in range(p.shape[1]):
+            acc = (acc.double() + p[:, r:r + 1].double() * q[r:r + 1].double()).float()
+        return acc
+
+    assert torch.equal(y.cpu(), chain(a, w2.t()))
+    assert torch.equal(dw.cpu(), chain(dy.t(), a))
+    assert torch.equal(dxs.cpu(), chain(dy, w2))
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.float64], ids=str)
 def test_generic_kernel_unaligned_operands(dt):
     """Operands one element past a 16-byte boundary (element loads) give the aligned operands' product."""
