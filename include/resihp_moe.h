@@ -311,6 +311,11 @@ int rhp_expert_fc1_fwd(int G, const int32_t* offsets, int rows_from_offsets, int
                        int h, int f, const void* const* xp, const void* const* w1, void* const* hpre,
                        void* const* act_out, void* split_ws, size_t split_ws_bytes, hipStream_t stream);
 
+/* The same product where no backward follows: only act leaves (a third of the rows' bytes for SwiGLU). */
+int rhp_expert_fc1_act(int G, const int32_t* offsets, int rows_from_offsets, int64_t rows_cap, int dtype, int act,
+                       int h, int f, const void* const* xp, const void* const* w1, void* const* act_out,
+                       void* split_ws, size_t split_ws_bytes, hipStream_t stream);
+
 /* y[r] = act[r] @ w2^T  ([M_g, h]). */
 int rhp_expert_fc2_fwd(int G, const int32_t* offsets, int rows_from_offsets, int64_t rows_cap, int dtype, int h,
                        int f, const void* const* act_in, const void* const* w2, void* const* y, void* split_ws,

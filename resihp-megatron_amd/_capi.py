@@ -48,6 +48,7 @@ SIGNATURES: dict[str, tuple[object, list]] = {
     "rhp_expert_split_workspace_reset": (_i, [_p, _sz, _p]),
     "rhp_expert_gemm_kernel": (_i, [_i, _i, _i, _i]),
     "rhp_expert_fc1_fwd": (_i, [_i, _p, _i, _i64, _i, _i, _i, _i, _pp, _pp, _pp, _pp, _p, _sz, _p]),
+    "rhp_expert_fc1_act": (_i, [_i, _p, _i, _i64, _i, _i, _i, _i, _pp, _pp, _pp, _p, _sz, _p]),
     "rhp_expert_fc2_fwd": (_i, [_i, _p, _i, _i64, _i, _i, _i, _pp, _pp, _pp, _p, _sz, _p]),
     "rhp_expert_fc2_bwd": (_i, [_i, _p, _i, _i64, _i, _i, _i, _i, _pp, _pp, _pp, _pp, _pp, _pp, _p, _sz, _p]),
     "rhp_expert_fc1_bwd": (_i, [_i, _p, _i, _i64, _i, _i, _i, _i, _pp, _pp, _pp, _pp, _pp, _p, _sz, _p]),

@@ -230,9 +230,9 @@ __device__ __forceinline__ void gg_bf16_tile(const Params& p, Tile t, uint8_t* l
             d64_kmaj(my, lda, wy * WY, FY, [&](int r) { return r < t.y_lim ? r : y_last; });
         }
         if (MODE == kFwd) {
-            rx = make_dma_rsrc(B, static_cast<int64_t>(EPI == kEpiSwigluFwd ? 2 * p.f : p.N) * p.ldb * 2);
+            rx = make_dma_rsrc(B, static_cast<int64_t>(is_swiglu_fwd(EPI) ? 2 * p.f : p.N) * p.ldb * 2);
             d64_kmaj(mx, ldb, wx * 128, 8, [&](int r) {
-                if (EPI == kEpiSwigluFwd) {
+                if (is_swiglu_fwd(EPI)) {
                     // 256 weight rows = [gate 64 | up 64] for each half of 128 activation columns.
                     const int half = r >> 7, qq = r & 127;
                     int col = t.x0 + half * 64 + (qq & 63);
@@ -541,9 +541,9 @@ __device__ __forceinline__ void gg_bf16_short_tile(const Params& p, Tile t, uint
         d64_kmaj(my, lda, 0, FY, [&](int r) { return r < t.y_lim ? r : y_last; });
     }
     if (MODE == kFwd) {
-        rx = make_dma_rsrc(B, static_cast<int64_t>(EPI == kEpiSwigluFwd ? 2 * p.f : p.N) * p.ldb * 2);
+        rx = make_dma_rsrc(B, static_cast<int64_t>(is_swiglu_fwd(EPI) ? 2 * p.f : p.N) * p.ldb * 2);
         d64_kmaj(mx, ldb, wave * 64, FX, [&](int r) {
-            if (EPI == kEpiSwigluFwd) {   // [gate 64 | up 64] for each half of 128 activation columns
+            if (is_swiglu_fwd(EPI)) {   // [gate 64 | up 64] for each half of 128 activation columns
                 const int half = r >> 7, qq = r & 127;
                 int col = t.x0 + half * 64 + (qq & 63);
                 col = col < p.f ? col : 0;
@@ -920,11 +920,13 @@ __global__ __launch_bounds__(256) void gg_generic_kernel(Params p) {
                 } else if (EPI == kEpiSwigluFwd) {
                     // the backward's factors [u silu'(g) | silu(g)] and the activation silu(g) u
                     const A up = acc[i][j + (EPI == kEpiSwigluFwd)][e], si = silu_f(v);
-                    Elem<S>::st(C, row * p.ldc + col, up * dsilu_f(v));
-                    Elem<S>::st(C, row * p.ldc + p.f + col, si);
+                    if (C) {   // null: only the activation leaves
+                        Elem<S>::st(C, row * p.ldc + col, up * dsilu_f(v));
+                        Elem<S>::st(C, row * p.ldc + p.f + col, si);
+                    }
                     Elem<S>::st(static_cast<S*>(p.c2[g]), row * p.ldc2 + col, si * up);
                 } else if (EPI == kEpiGeluFwd) {
-                    Elem<S>::st(C, row * p.ldc + col, v);
+                    if (C) Elem<S>::st(C, row * p.ldc + col, v);
                     Elem<S>::st(static_cast<S*>(p.c2[g]), row * p.ldc2 + col, gelu_f(v));
                 } else if (EPI == kEpiSwigluBwd) {
                     const S* hp = static_cast<const S*>(p.aux[g]);
@@ -1016,7 +1018,8 @@ void launch_one(const Job& j, const Params& p, hipStream_t s) {
         // A K split adds at most one round of pieces to each XCD's items.
         if (MODE != kWgrad && p.split_cap > 1) nb = kXcds * ((nb + kXcds - 1) / kXcds + p.cu_per_xcd);
         constexpr int nw = bf16_waves<MODE>();
-        if constexpr (MODE != kWgrad) {
+        constexpr bool kActOnly = EPI == kEpiSwigluAct || EPI == kEpiGeluAct;
+        if constexpr (MODE != kWgrad && !kActOnly) {
             if (j.a_idx || j.c_idx) {
                 hipLaunchKernelGGL((gg_bf16_kernel<MODE, EPI, nw, false, true>), dim3(static_cast<unsigned>(nb)),
                                    dim3(64 * nw), 0, s, p);
@@ -1036,9 +1039,11 @@ void launch_one(const Job& j, const Params& p, hipStream_t s) {
         hipLaunchKernelGGL((gg_bf16_kernel<MODE, EPI, nw>), dim3(static_cast<unsigned>(nb)), dim3(64 * nw), 0, s, p);
         return;
     }
-    if (j.dtype == RHP_BF16) launch_generic<bf16, MODE, EPI>(j, p, s);
-    else if (j.dtype == RHP_F32) launch_generic<float, MODE, EPI>(j, p, s);
-    else launch_generic<double, MODE, EPI>(j, p, s);
+    // The generic kernel's forward epilogues leave out the backward's values where c is null.
+    constexpr int GE = EPI == kEpiSwigluAct ? kEpiSwigluFwd : EPI == kEpiGeluAct ? kEpiGeluFwd : EPI;
+    if (j.dtype == RHP_BF16) launch_generic<bf16, MODE, GE>(j, p, s);
+    else if (j.dtype == RHP_F32) launch_generic<float, MODE, GE>(j, p, s);
+    else launch_generic<double, MODE, GE>(j, p, s);
 }
 
 void launch(const Job& j, const Params& p, hipStream_t s) {
@@ -1046,6 +1051,8 @@ void launch(const Job& j, const Params& p, hipStream_t s) {
         case kFwd * 8 + kEpiStore: launch_one<kFwd, kEpiStore>(j, p, s); break;
         case kFwd * 8 + kEpiSwigluFwd: launch_one<kFwd, kEpiSwigluFwd>(j, p, s); break;
         case kFwd * 8 + kEpiGeluFwd: launch_one<kFwd, kEpiGeluFwd>(j, p, s); break;
+        case kFwd * 8 + kEpiSwigluAct: launch_one<kFwd, kEpiSwigluAct>(j, p, s); break;
+        case kFwd * 8 + kEpiGeluAct: launch_one<kFwd, kEpiGeluAct>(j, p, s); break;
         case kDgrad * 8 + kEpiStore: launch_one<kDgrad, kEpiStore>(j, p, s); break;
         case kDgrad * 8 + kEpiSwigluBwd: launch_one<kDgrad, kEpiSwigluBwd>(j, p, s); break;
         case kDgrad * 8 + kEpiGeluBwd: launch_one<kDgrad, kEpiGeluBwd>(j, p, s); break;
@@ -1084,7 +1091,7 @@ int run(const Job& job, const char* what, hipStream_t s) {
         for (int i = 0; i < gn; ++i) {
             p.a[i] = j.a[g0 + i];
             p.b[i] = j.b[g0 + i];
-            p.c[i] = j.c[g0 + i];
+            p.c[i] = j.c ? j.c[g0 + i] : nullptr;
             p.c2[i] = j.c2 ? j.c2[g0 + i] : nullptr;
             p.aux[i] = j.aux ? j.aux[g0 + i] : nullptr;
         }
@@ -1199,23 +1206,23 @@ extern "C" int rhp_expert_gemm_kernel(int dtype, int act, int h, int f) {
     return mfma_shape_ok(dtype, h, f, act) ? RHP_GEMM_KERNEL_MFMA : RHP_GEMM_KERNEL_GENERIC;
 }
 
-extern "C" int rhp_expert_fc1_fwd(int G, const int32_t* offsets, int rows_from_offsets, int64_t rows_cap, int dtype,
-                                  int act, int h, int f, const void* const* xp, const void* const* w1,
-                                  void* const* hpre, void* const* act_out, void* split_ws, size_t split_ws_bytes,
-                                  hipStream_t stream) {
-    clear_error();
-    if (int rc = check_common("rhp_expert_fc1_fwd", G, offsets, rows_cap, dtype, act, h, f)) return rc;
-    if (int rc = check_split_ws("rhp_expert_fc1_fwd", split_ws, split_ws_bytes)) return rc;
-    RHP_REQUIRE(all_set(xp, G) && all_set(w1, G) && all_set((const void* const*)hpre, G) &&
-                    all_set((const void* const*)act_out, G),
-                "rhp_expert_fc1_fwd: null pointer");
+namespace rhp {
+namespace {
+// fc1's forward product; hpre null: only the activation rows are written.
+int fc1_forward(const char* fn, int G, const int32_t* offsets, int rows_from_offsets, int64_t rows_cap, int dtype,
+                int act, int h, int f, const void* const* xp, const void* const* w1, void* const* hpre,
+                void* const* act_out, void* split_ws, size_t split_ws_bytes, hipStream_t stream) {
+    if (int rc = check_common(fn, G, offsets, rows_cap, dtype, act, h, f)) return rc;
+    if (int rc = check_split_ws(fn, split_ws, split_ws_bytes)) return rc;
+    if (!all_set(xp, G) || !all_set(w1, G) || (hpre && !all_set((const void* const*)hpre, G)) ||
+        !all_set((const void* const*)act_out, G))
+        return fail(std::string(fn) + ": null pointer");
     const bool swiglu = act == RHP_ACT_SWIGLU;
-    const int F1 = swiglu ? 2 * f : f;
     Job j{};
     j.mode = kFwd;
-    j.epi = swiglu ? kEpiSwigluFwd : kEpiGeluFwd;
+    j.epi = hpre ? (swiglu ? kEpiSwigluFwd : kEpiGeluFwd) : (swiglu ? kEpiSwigluAct : kEpiGeluAct);
     j.dtype = dtype;
-    if (int rc = choose_kernel("rhp_expert_fc1_fwd", dtype, h, f, act,
+    if (int rc = choose_kernel(fn, dtype, h, f, act,
                                all_aligned(xp, G) && all_aligned(w1, G) && all_aligned((const void* const*)hpre, G) &&
                                    all_aligned((const void* const*)act_out, G),
                                &j.mfma))
@@ -1228,7 +1235,7 @@ extern "C" int rhp_expert_fc1_fwd(int G, const int32_t* offsets, int rows_from_o
     j.K = h;
     j.lda = h;
     j.ldb = h;
-    j.ldc = F1;
+    j.ldc = swiglu ? 2 * f : f;
     j.ldc2 = f;
     j.f = f;
     j.a = xp;
@@ -1236,7 +1243,27 @@ extern "C" int rhp_expert_fc1_fwd(int G, const int32_t* offsets, int rows_from_o
     j.c = hpre;
     j.c2 = act_out;
     j.split_ws = split_ws;
-    return run(j, "expert_fc1_fwd", stream);
+    return run(j, fn, stream);
+}
+}  // namespace
+}  // namespace rhp
+
+extern "C" int rhp_expert_fc1_fwd(int G, const int32_t* offsets, int rows_from_offsets, int64_t rows_cap, int dtype,
+                                  int act, int h, int f, const void* const* xp, const void* const* w1,
+                                  void* const* hpre, void* const* act_out, void* split_ws, size_t split_ws_bytes,
+                                  hipStream_t stream) {
+    clear_error();
+    RHP_REQUIRE(hpre != nullptr, "rhp_expert_fc1_fwd: null pointer");
+    return fc1_forward("rhp_expert_fc1_fwd", G, offsets, rows_from_offsets, rows_cap, dtype, act, h, f, xp, w1, hpre,
+                       act_out, split_ws, split_ws_bytes, stream);
+}
+
+extern "C" int rhp_expert_fc1_act(int G, const int32_t* offsets, int rows_from_offsets, int64_t rows_cap, int dtype,
+                                  int act, int h, int f, const void* const* xp, const void* const* w1,
+                                  void* const* act_out, void* split_ws, size_t split_ws_bytes, hipStream_t stream) {
+    clear_error();
+    return fc1_forward("rhp_expert_fc1_act", G, offsets, rows_from_offsets, rows_cap, dtype, act, h, f, xp, w1, nullptr,
+                       act_out, split_ws, split_ws_bytes, stream);
 }
 
 extern "C" int rhp_expert_fc2_fwd(int G, const int32_t* offsets, int rows_from_offsets, int64_t rows_cap, int dtype,

@@ -547,6 +547,20 @@ def expert_fc1_fwd(xs: list[torch.Tensor], offsets: torch.Tensor, rows_from_offs
                 dtype_code(w1[0]), act_code(act), h, f, _arr(xs), _arr(w1), _arr(hpre), _arr(act_out))
 
 
+def expert_fc1_act(xs: list[torch.Tensor], offsets: torch.Tensor, rows_from_offsets: bool, rows_cap: int,
+                   w1: list[torch.Tensor], f: int, act: str, act_out: list[torch.Tensor], split: bool = True) -> None:
+    """expert_fc1_fwd where no backward follows: only the activation rows are written."""
+    dev = _need_cuda(offsets, xs, w1, act_out)
+    G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
+    rows = _shared_rows(rows_from_offsets, rows_cap)
+    _check_offsets(offsets, G)
+    _check_groups("w1", w1, G, dt, h, exact_shape=(2 * f if act == "swiglu" else f, h))
+    _check_groups("x", xs, G, dt, h, rows)
+    _check_groups("act", act_out, G, dt, f, rows)
+    _split_call("rhp_expert_fc1_act", dev, split, G, _ptr(offsets), int(rows_from_offsets), rows_cap,
+                dtype_code(w1[0]), act_code(act), h, f, _arr(xs), _arr(w1), _arr(act_out))
+
+
 def expert_fc2_fwd(acts: list[torch.Tensor], offsets: torch.Tensor, rows_from_offsets: bool, rows_cap: int,
                    w2: list[torch.Tensor], ys: list[torch.Tensor], split: bool = True) -> None:
     dev = _need_cuda(offsets, acts, w2, ys)

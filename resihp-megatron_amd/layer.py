@@ -193,9 +193,21 @@ def _fp8_backward(st: Fp8State, q8: dict, meta: LayerMeta, offsets, P, dyq, hpre
                s[X:X + 1])
 
 
+def _fc1_fwd(xs, offsets, rows_from_offsets: bool, rows_cap: int, fc1s, f: int, act: str, hpres, acts) -> None:
+    """fc1's forward product; ``hpres`` None: without what a backward needs."""
+    if hpres is None:
+        K.expert_fc1_act(xs, offsets, rows_from_offsets, rows_cap, fc1s, f, act, acts)
+    else:
+        K.expert_fc1_fwd(xs, offsets, rows_from_offsets, rows_cap, fc1s, f, act, hpres, acts)
+
+
 class _MoELayerFn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, meta: LayerMeta, fp8, x, router_w, bias, *weights):
+    def forward(ctx, meta: LayerMeta, opts, x, router_w, bias, *weights):
+        fp8, grad_mode = opts
+        # Without a backward to come (no_grad, or no input that needs a gradient) fc1 writes only the
+        # activation rows, and nothing is saved.
+        keep = fp8 is not None or (grad_mode and any(ctx.needs_input_grad))
         e0, e1 = meta.window
         G = e1 - e0
         S = meta.num_shared
@@ -212,14 +224,14 @@ class _MoELayerFn(torch.autograd.Function):
         shared_side = S > 0 and T > 0 and _concurrent(h, _fc1_rows(meta.act, fs))
         if S:
             shared_off = torch.arange(S + 1, dtype=torch.int32, device=x.device) * T
-            shared_h = [x.new_empty(T, _fc1_rows(meta.act, fs)) for _ in range(S)]
+            shared_h = [x.new_empty(T, _fc1_rows(meta.act, fs)) for _ in range(S)] if keep else None
             shared_a = [x.new_empty(T, fs) for _ in range(S)]
             shared_y = [x.new_empty(T, h) for _ in range(S)]
         if shared_side:
             side = _side_stream(x.device)
             side.wait_stream(main)
             with torch.cuda.stream(side):
-                K.expert_fc1_fwd([x] * S, shared_off, False, T, sfc1s, fs, meta.act, shared_h, shared_a)
+                _fc1_fwd([x] * S, shared_off, False, T, sfc1s, fs, meta.act, shared_h, shared_a)
                 K.expert_fc2_fwd(shared_a, shared_off, False, T, sfc2s, shared_y)
         # fp8 experts (never with shared experts): the weight casts start now, on the side stream.
         wcast = _fp8_weight_casts(fp8, weights[:G], weights[G:2 * G], main) if fp8 is not None else None
@@ -231,7 +243,7 @@ class _MoELayerFn(torch.autograd.Function):
         F1 = _fc1_rows(meta.act, f)
         # fp8 experts read only the input rows' codes: the permute writes them instead of bf16 rows.
         xp = K.permute(x, plan.pair_row, k, P) if fp8 is None else x.new_empty(0, h)
-        hpre = x.new_empty(P, F1)
+        hpre = x.new_empty(P, F1) if keep else None
         act = x.new_empty(0 if fp8 is not None else P, f)   # the fp8 path keeps only the activation's codes
         y = x.new_empty(P, h)
         q8 = None
@@ -240,21 +252,23 @@ class _MoELayerFn(torch.autograd.Function):
             q8 = _fp8_forward(fp8, meta, plan.offsets, P, xq, fc1s, fc2s, hpre, y, wcast)
             q8["xq"] = xq
         elif P > 0:
-            K.expert_fc1_fwd([xp] * G, plan.offsets, True, P, fc1s, f, meta.act, [hpre] * G, [act] * G)
+            _fc1_fwd([xp] * G, plan.offsets, True, P, fc1s, f, meta.act, [hpre] * G if keep else None, [act] * G)
             K.expert_fc2_fwd([act] * G, plan.offsets, True, P, fc2s, [y] * G)
         if S and T > 0 and not shared_side:
-            K.expert_fc1_fwd([x] * S, shared_off, False, T, sfc1s, fs, meta.act, shared_h, shared_a)
+            _fc1_fwd([x] * S, shared_off, False, T, sfc1s, fs, meta.act, shared_h, shared_a)
             K.expert_fc2_fwd(shared_a, shared_off, False, T, sfc2s, shared_y)
         if shared_side:
             main.wait_stream(_side_stream(x.device))
         out = K.combine(y, x, gates, topi, plan.pair_row, shared_y or [])
+        ctx.mark_non_differentiable(plan.counts)
+        if not keep:
+            return out, plan.counts
         ctx.meta = meta
         ctx.fp8 = (fp8, q8)
         ctx.dims = (T, h, P, G, S)
         ctx.save_for_backward(x, router_w, logits, topi, gates, plan.perm, plan.offsets, plan.pair_row, xp, hpre,
                               act, y, *weights)
         ctx.shared = (shared_off, shared_h, shared_a)
-        ctx.mark_non_differentiable(plan.counts)
         return out, plan.counts
 
     @staticmethod
@@ -457,6 +471,6 @@ def moe_layer(meta: LayerMeta, x: torch.Tensor, router_w: torch.Tensor, bias: to
         raise ValueError(f"need one fc1 and one fc2 weight per local expert ({e1 - e0})")
     if len(shared_fc1s) != meta.num_shared or len(shared_fc2s) != meta.num_shared:
         raise ValueError(f"need {meta.num_shared} shared expert weight pairs")
-    return _MoELayerFn.apply(meta, fp8, x.contiguous(), router_w.contiguous(),
+    return _MoELayerFn.apply(meta, (fp8, torch.is_grad_enabled()), x.contiguous(), router_w.contiguous(),
                              None if bias is None else bias.detach().contiguous(),
                              *fc1s, *fc2s, *shared_fc1s, *shared_fc2s)

@@ -321,6 +321,40 @@ def test_config5_fp8_full_size():
     _full_size_layer("c5-fp8", 16384, 4096, 14336, 8, 2, fp8=True)
 
 
+@pytest.mark.parametrize("T,h,f,E,k,S,act,dt,window", [
+    (37, 256, 192, 8, 2, 1, "swiglu", torch.bfloat16, None),        # few rows a group: short tiles
+    (700, 256, 192, 4, 2, 2, "swiglu", torch.bfloat16, None),       # whole and ragged tiles, a half column tile
+    (9, 2048, 128, 4, 2, 0, "swiglu", torch.bfloat16, None),        # K split of the few-row launch
+    (300, 128, 320, 4, 1, 1, "gelu", torch.bfloat16, None),
+    (300, 128, 192, 8, 2, 0, "swiglu", torch.bfloat16, (2, 6)),     # a window of the experts
+    (129, 72, 51, 6, 2, 1, "swiglu", torch.float32, None),          # generic kernel
+    (129, 72, 50, 6, 2, 0, "gelu", torch.float64, None),
+])
+def test_forward_without_backward_is_the_same(T, h, f, E, k, S, act, dt, window):
+    """Where no gradient is wanted the forward keeps nothing for one; its output is the same, bit for bit."""
+    e0, e1 = window or (0, E)
+    F1 = 2 * f if act == "swiglu" else f
+    d = lambda t: t.to(DEV)  # noqa: E731
+    x = d(seeded((T, h), 1, 1.0, dt))
+    router = d(seeded((E, h), 2, 0.1, torch.float64 if dt == torch.float64 else torch.float32))
+    fc1, fc2 = ([d(seeded(s, seed + e, 0.05, dt)) for e in range(e0, e1)] for s, seed in (((F1, h), 10), ((h, f), 40)))
+    s1, s2 = ([d(seeded(s, seed + e, 0.05, dt)) for e in range(S)] for s, seed in (((F1, h), 70), ((h, f), 90)))
+    meta = LayerMeta(num_experts=E, top_k=k, ffn=f, act=act, e0=e0, e1=e1, num_shared=S)
+    say(f"no-grad forward T={T} h={h} f={f} E={E} {act} {dt}")
+    args = (meta, x, router, None, fc1, fc2, s1, s2)
+    plain, counts = moe_layer(*args)   # no input wants a gradient
+    assert plain.grad_fn is None
+    fc1[-1].requires_grad_(True)
+    with torch.no_grad():
+        quiet, _ = moe_layer(*args)
+    out, ref_counts = moe_layer(*args)
+    assert out.requires_grad and not quiet.requires_grad
+    torch.cuda.synchronize()
+    assert torch.equal(plain, out) and torch.equal(quiet, out) and torch.equal(counts, ref_counts)
+    out.sum().backward()
+    assert fc1[-1].grad is not None
+
+
 def test_reference_default_gelu_fp64():
     _run("reference-default", moe.MoEConfig(device=DEV), check_route=True)
 
