@@ -33,16 +33,17 @@ namespace {
 
 constexpr int kAdamMax = 64;        // tensors per launch
 constexpr int kAdamThreads = 256;
-// Elements per thread.  One 8-element group of each of the four arrays, all
-// loads and stores non-temporal (nothing is read twice): the step is bound by
-// HBM, and small blocks that come and go keep its reads and writes mixed.
+// Elements per thread: 16 bytes of each of the four arrays, all loads and
+// stores non-temporal (nothing is read twice): the step is bound by HBM, and
+// small blocks that come and go keep its reads and writes mixed.
 // 1.41 G bfloat16 parameters (14 bytes each, 256 threads a block): 4 groups a
 // thread with ordinary accesses 3664 us, 5.39 TB/s; non-temporal 3479; 2
 // groups 3487; 1 group 3305, 5.97 TB/s (ordinary accesses 3573).  Cutting a
 // quarter of the instructions (shorter exact square root and divisions)
 // changed none of these by more than 2 %, so the plain forms stay.
-constexpr int kAdamElems = 8;
-constexpr int64_t kAdamBlockElems = int64_t(kAdamThreads) * kAdamElems;
+// Wider types take as many bytes, not as many elements: @F32@
+template <class S> constexpr int kAdamElems = 16 / static_cast<int>(sizeof(S));
+template <class S> constexpr int64_t kAdamBlockElems = int64_t(kAdamThreads) * kAdamElems<S>;
 
 struct AdamTensors {
     void* p[kAdamMax];
@@ -150,20 +151,13 @@ __device__ __forceinline__ void adam_two_bf16(const AdamScalars<float>& sc, floa
     round2(p[0], p[1]);
 }
 
-// Raw 16-byte groups of 8 elements.
-template <class S> struct Group8 {
+// A thread's 16 bytes of one array.
+template <class S> struct Group {
     typedef uint32_t Word __attribute__((ext_vector_type(4)));
-    static constexpr int kWords = static_cast<int>(sizeof(S)) * 8 / 16;
-    Word w[kWords];
-    __device__ __forceinline__ void load(const S* p) {
-#pragma unroll
-        for (int i = 0; i < kWords; ++i) w[i] = __builtin_nontemporal_load(reinterpret_cast<const Word*>(p) + i);
-    }
-    __device__ __forceinline__ void store(S* p) const {
-#pragma unroll
-        for (int i = 0; i < kWords; ++i) __builtin_nontemporal_store(w[i], reinterpret_cast<Word*>(p) + i);
-    }
-    __device__ __forceinline__ S& at(int e) { return reinterpret_cast<S*>(w)[e]; }
+    Word w;
+    __device__ __forceinline__ void load(const S* p) { w = __builtin_nontemporal_load(reinterpret_cast<const Word*>(p)); }
+    __device__ __forceinline__ void store(S* p) const { __builtin_nontemporal_store(w, reinterpret_cast<Word*>(p)); }
+    __device__ __forceinline__ S& at(int e) { return reinterpret_cast<S*>(&w)[e]; }
 };
 
 template <class S> __device__ __forceinline__ typename AdamElem<S>::T to_t(S x);
@@ -176,11 +170,12 @@ template <> __device__ __forceinline__ float from_t<float>(float x) { return x; 
 template <> __device__ __forceinline__ bf16 from_t<bf16>(float x) { return bf16{AdamElem<bf16>::bits(x)}; }
 
 // Block b updates elements [B * (b - block0[t]), +B) of tensor t, B =
-// kAdamBlockElems: each thread 8 consecutive elements, all loads issued before
-// the first update.
+// kAdamBlockElems: each thread kAdamElems consecutive elements, all loads issued
+// before the first update.
 template <class S>
 __global__ __launch_bounds__(kAdamThreads) void adam_kernel(AdamTensors ts, AdamScalars<typename AdamElem<S>::T> sc) {
     using T = typename AdamElem<S>::T;
+    constexpr int kN = kAdamElems<S>;
     // The block's tensor: one candidate per lane (a scalar load per tensor in turn took longer than the update).
     static_assert(kAdamMax <= 64, "one tensor per lane");
     const int lane = static_cast<int>(threadIdx.x & 63);
@@ -191,16 +186,16 @@ __global__ __launch_bounds__(kAdamThreads) void adam_kernel(AdamTensors ts, Adam
     const S* G = static_cast<const S*>(ts.g[t]);
     S* M = static_cast<S*>(ts.m[t]);
     S* V = static_cast<S*>(ts.v[t]);
-    const int64_t e0 = static_cast<int64_t>(blockIdx.x - ts.block0[t]) * kAdamBlockElems + threadIdx.x * kAdamElems;
-    if (e0 < n / 8 * 8) {   // a whole 8-element group
-        Group8<S> gp, gg, gm, gv;
+    const int64_t e0 = static_cast<int64_t>(blockIdx.x - ts.block0[t]) * kAdamBlockElems<S> + threadIdx.x * kN;
+    if (e0 < n / kN * kN) {   // a whole group
+        Group<S> gp, gg, gm, gv;
         gp.load(P + e0);
         gm.load(M + e0);
         gv.load(V + e0);
         if (G) gg.load(G + e0);
         if constexpr (std::is_same<S, bf16>::value) {
 #pragma unroll
-            for (int e = 0; e < 8; e += 2) {
+            for (int e = 0; e < kN; e += 2) {
                 float p[2], g[2], m[2], v[2];
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
@@ -219,7 +214,7 @@ __global__ __launch_bounds__(kAdamThreads) void adam_kernel(AdamTensors ts, Adam
             }
         } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
+            for (int e = 0; e < kN; ++e) {
                 T p = to_t<S>(gp.at(e)), m = to_t<S>(gm.at(e)), v = to_t<S>(gv.at(e));
                 const T g = G ? to_t<S>(gg.at(e)) : T(0);
                 adam_one<S>(sc, p, g, m, v);
@@ -258,7 +253,7 @@ int launch_adam(int count, void* const* params, const void* const* grads, void* 
             ts.v[i] = v[t0 + i];
             ts.n[i] = numel[t0 + i];
             ts.block0[i] = static_cast<uint32_t>(blocks);
-            blocks += static_cast<uint64_t>((numel[t0 + i] + kAdamBlockElems - 1) / kAdamBlockElems);
+            blocks += static_cast<uint64_t>((numel[t0 + i] + kAdamBlockElems<S> - 1) / kAdamBlockElems<S>);
         }
         ts.block0[ts.count] = static_cast<uint32_t>(blocks);
         RHP_REQUIRE(blocks < (uint64_t(1) << 31), "rhp_adam_step: too many elements in one launch");
