@@ -41,7 +41,8 @@ constexpr int kAdamThreads = 256;
 // groups 3487; 1 group 3305, 5.97 TB/s (ordinary accesses 3573).  Cutting a
 // quarter of the instructions (shorter exact square root and divisions)
 // changed none of these by more than 2 %, so the plain forms stay.
-// Wider types take as many bytes, not as many elements: @F32@
+// Wider types take as many bytes, not as many elements, so that a wave's
+// access is whole lines: 8.6 M float32 parameters 46.6 us with 8 a thread, 40.2.
 template <class S> constexpr int kAdamElems = 16 / static_cast<int>(sizeof(S));
 template <class S> constexpr int64_t kAdamBlockElems = int64_t(kAdamThreads) * kAdamElems<S>;
 
