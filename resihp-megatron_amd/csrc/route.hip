@@ -494,6 +494,98 @@ __device__ __forceinline__ void load_block_ids(const int32_t* topi, int64_t p0, 
     }
 }
 
+// The whole plan of one source's at most kDispatchPairs pairs in one block, in
+// place of the three kernels below: with so few pairs they are launch latency
+// (kernel time, 8 tokens by 2 slots, 8 experts: 10.5 us in three launches, 3.2 in
+// one; 64 by 6, 64 experts: 17.3 and 5.1; 2048 by 2, 8 experts: 19.3 and 13.3;
+// 512 by 8, 128 experts: 27.1 and 20.0).  Wave w
+// takes the w-th quarter of the pairs, in order, so ranks need no exchange
+// between waves beyond one scan: it counts its pairs per expert, the block
+// turns the counts into each wave's first place within each expert and the
+// experts' first rows, and each wave then places its pairs, 64 at a time.
+// More pairs keep the kernels below, whose blocks share the work.  256 threads
+// for the reason given at dispatch_scan_kernel.
+__global__ __launch_bounds__(kThreads) void dispatch_one_block_kernel(const int32_t* __restrict__ topi, DispatchShape d,
+                                                                      int32_t* __restrict__ counts,
+                                                                      int32_t* __restrict__ offsets,
+                                                                      int32_t* __restrict__ src_counts,
+                                                                      int32_t* __restrict__ perm,
+                                                                      int32_t* __restrict__ pair_row) {
+    constexpr int kWaves = kThreads / 64, kRounds = kDispatchPairs / kThreads;
+    __shared__ int place[kWaves][kMaxE + 1];   // pairs of (wave, expert), then the next place in the expert
+    __shared__ int tot[kMaxE + 1];
+    __shared__ int off[kMaxE];
+    const int L = d.e1 - d.e0;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int P = static_cast<int>(d.T) * d.k;
+    const int rounds = (P + kThreads - 1) / kThreads, p0 = wave * rounds * 64 + lane;
+    int ids[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int p = p0 + r * 64;
+        const int e = r < rounds && p < P ? topi[p] : -1;
+        ids[r] = e < 0 || e >= d.E ? d.E : e;   // d.E counts ids outside [0, E)
+    }
+    for (int e = lane; e <= d.E; e += 64) place[wave][e] = 0;
+    const int nbits = key_bits(d.E + 1);
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        if (r >= rounds) break;
+        const uint64_t m = match_any(p0 + r * 64 < P, ids[r], nbits);
+        if (m && (m & lanemask_lt(lane)) == 0) atomicAdd(&place[wave][ids[r]], __popcll(m));
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e <= d.E; e += kThreads) {
+        int sum = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const int c = place[w][e];
+            place[w][e] = sum;
+            sum += c;
+        }
+        tot[e] = sum;
+        counts[e] = sum;
+    }
+    __syncthreads();
+    if (wave == 0) {   // the local experts' first rows, 64 experts at a time
+        int run = 0;
+        for (int i0 = 0; i0 < L; i0 += 64) {
+            const int i = i0 + lane, c = i < L ? tot[d.e0 + i] : 0;
+            int incl = c;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int up = __shfl_up(incl, o, 64);
+                if (lane >= o) incl += up;
+            }
+            if (i < L) {
+                off[i] = run + incl - c;
+                offsets[i] = run + incl - c;
+                src_counts[i] = c;
+            }
+            run += __shfl(incl, 63, 64);
+        }
+        if (lane == 0) offsets[L] = run;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        if (r >= rounds) break;
+        const int p = p0 + r * 64, e = ids[r];
+        const bool local = p < P && e >= d.e0 && e < d.e1;
+        const uint64_t m = match_any(local, e, nbits);
+        const int rank = __popcll(m & lanemask_lt(lane));
+        int first = 0;
+        if (local && rank == 0) first = off[e - d.e0] + atomicAdd(&place[wave][e], __popcll(m));
+        first = __shfl(first, local ? __ffsll(static_cast<unsigned long long>(m)) - 1 : lane, 64);
+        if (local) {
+            perm[first + rank] = p;
+            pair_row[p] = first + rank;
+        } else if (p < P) {
+            pair_row[p] = -1;
+        }
+    }
+}
+
 // Phase 1: per-block expert histogram; one LDS atomic per distinct id of a wave and round.
 __global__ __launch_bounds__(kThreads) void dispatch_count_kernel(const int32_t* __restrict__ topi, DispatchShape d,
                                                                   int32_t* __restrict__ block_counts,
@@ -829,8 +921,8 @@ extern "C" size_t rhp_dispatch_workspace_bytes(int64_t T, int k, int E, int n_sr
 namespace rhp {
 namespace {
 
-// The dispatch plan with its workspace: argument checks, then the count,
-// scan and scatter kernels.  Every launch writes each workspace entry it
+// The dispatch plan with its workspace: argument checks, then the one-block
+// kernel (few pairs of one source) or the count, scan and scatter kernels.  Every launch writes each workspace entry it
 // reads (per-block histograms, sources and base rows), so the workspace
 // needs no clearing.
 int dispatch_run(const char* fn, const int32_t* topi, int64_t T, int k, int E, int e0, int e1, int n_src,
@@ -853,6 +945,11 @@ int dispatch_run(const char* fn, const int32_t* topi, int64_t T, int k, int E, i
     d.e1 = e1;
     d.n_src = n_src;
     d.nblk = dispatch_blocks(T, k, n_src, &d.tokens_per_block);
+    if (n_src == 1 && T > 0 && T * k <= kDispatchPairs) {
+        hipLaunchKernelGGL(dispatch_one_block_kernel, dim3(1), dim3(kThreads), 0, stream, topi, d, counts, offsets,
+                           src_counts, perm, pair_row);
+        return check_launch("dispatch_one_block_kernel");
+    }
     const int L = e1 - e0;
     int32_t* block_counts = static_cast<int32_t*>(workspace);
     int32_t* block_base = block_counts + static_cast<size_t>(d.nblk) * (E + 1);

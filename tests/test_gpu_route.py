@@ -162,6 +162,28 @@ def test_dispatch_bit_exact(case):
         assert (ref["counts"][list(EMPTY)] == 0).all() and P > 0
 
 
+@pytest.mark.parametrize("T,k,E,e0,e1", [
+    (2048, 2, 8, 0, 8), (1365, 3, 64, 5, 63), (1366, 3, 64, 5, 63), (64, 1, 1, 0, 1), (65, 1, 1024, 0, 1024),
+    (511, 8, 130, 0, 130), (43, 6, 64, 0, 64), (257, 1, 7, 6, 7),
+])
+def test_dispatch_few_pairs(T, k, E, e0, e1):
+    """The one-block plan at the ends of its range (up to 4096 pairs), of a wave's and of a round's pairs, with
+    ids outside [0, E) and a window of the experts, and the first size past it."""
+    g = torch.Generator().manual_seed(T)
+    topi = _topi(T, min(k, E), E, 1.0, 11)
+    topi[torch.rand(topi.shape, generator=g) < 0.05] = E + 3
+    topi[torch.rand(topi.shape, generator=g) < 0.05] = -1
+    say(f"dispatch few pairs T={T} k={k} E={E} window=[{e0},{e1})")
+    plan = K.dispatch(topi.to(DEV), E, e0, e1)
+    torch.cuda.synchronize()
+    ref = R.dispatch(topi.numpy(), E, e0, e1)
+    assert np.array_equal(plan.counts.cpu().numpy(), ref["counts"])
+    assert np.array_equal(plan.offsets.cpu().numpy(), ref["offsets"])
+    assert np.array_equal(plan.src_counts.cpu().numpy(), ref["src_counts"])
+    assert np.array_equal(plan.perm[:int(ref["offsets"][-1])].cpu().numpy(), ref["perm"])
+    assert np.array_equal(plan.pair_row.cpu().numpy(), ref["pair_row"])
+
+
 def test_dispatch_invalid_ids_dropped():
     topi = torch.tensor([[0, 9], [-1, 1], [3, 2]], dtype=torch.int32)
     say("dispatch invalid ids")
