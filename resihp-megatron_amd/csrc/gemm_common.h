@@ -54,7 +54,6 @@ struct Params {
     int32_t* split_cnt;       // [8 * cu_per_xcd] arrival counters, zero between launches
     int split_cap;
     int cu_per_xcd;
-    int split_piece_k;        // reduction length a piece keeps at least
     int split_kstep;          // the kernel's K step: pieces start and end on multiples of it
     // Quantising epilogues (fp8 kernels): the activation (forward) or the
     // pre-activation gradient (backward) leaves as fp8 codes instead of bf16,
@@ -144,16 +143,13 @@ constexpr int kXcds = 8;
 // A split pays only where a tile's reduction is long: each piece publishes
 // a 256 KB partial tile behind an L2-wide release, and the last one reads all
 // of them back.  Measured at K = 1408-4096 the split lost up to 8 %, at
-// K = 14336 and 28672 it gained 4 % and 2 %.  Where groups hold few rows the
-// partial tiles are only the 16-row fragments that hold any, and the launch
-// streams weights: its time is its rounds of tiles, and a last round of a few
-// tiles costs a whole one unless they are split (8 experts of 4096 by 14336, 8
-// tokens, 806 fc1 tiles on 256 CUs).
+// K = 14336 and 28672 it gained 4 % and 2 %.  The line does not depend on how
+// many rows a launch holds: below it every output is one chain over k, the same
+// bits whatever rows share its launch.  (Launches of at most 64 rows a group
+// gained up to 6 % of a product from a split at K = 2048 and 4096, but a row's
+// last bits then changed with its batch.)
 constexpr int kSplitMinK = 8192;        // reduction length a tile needs to be split at all
 constexpr int kSplitMinPieceK = 1024;   // reduction length a split piece keeps at least
-constexpr int kSplitFewRows = 64;       // average rows a group up to which the lengths below hold instead
-constexpr int kSplitFewMinK = 2048;
-constexpr int kSplitFewPieceK = 512;
 
 // K-split workspace: 8 XCDs x up to kSplitMaxCus pieces of one fp32 tile each,
 // then one arrival counter per piece slot.
@@ -270,9 +266,9 @@ __device__ __forceinline__ int find_tile(const Params& p, int xt_cols, int yt_ro
         const uint32_t q = total / kXcds, r = total % kXcds;
         const uint32_t n = q + (x < r ? 1u : 0u), start = x * q + (x < r ? x : r);
         const uint32_t F = n / C * C, rx = n - F;
-        uint32_t s = rx ? C / rx : 1u;   // (the host sets split_cap only for reductions that may be split)
+        uint32_t s = rx && p.K >= kSplitMinK ? C / rx : 1u;
         s = min(s, static_cast<uint32_t>(p.split_cap));
-        s = min(s, static_cast<uint32_t>(p.K / p.split_piece_k));
+        s = min(s, static_cast<uint32_t>(p.K / kSplitMinPieceK));
         if (j < F || s < 2) {
             if (j >= n) return kTileDone;
             L = start + j;

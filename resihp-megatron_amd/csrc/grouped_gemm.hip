@@ -498,10 +498,11 @@ __device__ __forceinline__ void gg_bf16_tile(const Params& p, Tile t, uint8_t* l
 // 128 rows, half the loads; each block of 32 MFMAs carries 12 fragment reads
 // (forward; 16 with the input gradients' half-reads) and 8 or 4 loads, one
 // memory instruction after each of its first MFMAs, loads spread evenly.
-//   Bound by the weights' HBM traffic; with the K split of few-row launches
-// (kSplitFewRows), 8 tokens by 8 experts of 4096 by 14336: fc1 forward 374 ->
-// 310 us (4.5 -> 5.4 TB/s), fc2 forward 211 -> 149 (4.0 -> 5.7); 64 tokens by 64
-// experts of 2048 by 1408, top 6: 155 -> 125 and 71 -> 60 us.
+//   Bound by the weights' HBM traffic and, where a launch has only a few rounds
+// of tiles, by its last, partly filled one.  8 tokens by 8 experts of 4096 by
+// 14336: fc1 forward 346 -> 308 us, fc2 forward (its last round split along K)
+// 200 -> 143; 64 tokens by 64 experts of 2048 by 1408, top 6: 152 -> 127 and
+// 72 -> 59 us.
 template <int MODE, int EPI, bool MAP>
 __device__ __forceinline__ void gg_bf16_short_tile(const Params& p, Tile t, uint8_t* lds) {
     constexpr int NW = 4, FX = 4, FY = 8;
@@ -1118,14 +1119,12 @@ int run(const Job& job, const char* what, hipStream_t s) {
         p.rw_e0 = j.rw_e0 + g0;
         // Only reductions long enough to be split get the split (and its larger
         // grid: the extra, mostly empty blocks cost about 1 % of a short product).
-        const bool few = j.rows_cap <= static_cast<int64_t>(kSplitFewRows) * (j.rows_from_offsets ? gn : 1);
-        if (j.split_ws && j.mfma && j.mode != kWgrad && j.K >= (few ? kSplitFewMinK : kSplitMinK)) {
+        if (j.split_ws && j.mfma && j.mode != kWgrad && j.K >= kSplitMinK) {
             const int C = std::min(kSplitMaxCus, j.cus_per_xcd);
             if (C > 1) {
                 p.split_part = static_cast<float*>(j.split_ws);
                 p.split_cnt = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(j.split_ws) + kSplitPartBytes);
                 p.split_cap = kSplitCap;
-                p.split_piece_k = few ? kSplitFewPieceK : kSplitMinPieceK;
                 p.cu_per_xcd = C;
                 p.split_kstep = 64;
             }

@@ -113,13 +113,17 @@ def test_grouped_expert_gemms(case, act):
 
 
 # Groups of few rows on the bf16 kernel: tiles of at most 128 rows (1, a fragment and its neighbours, 127, 128;
-# 129 takes a full tile), and their reduction split along K (at most 64 rows a group on average, from 2048),
-# also beside one group of several full tiles.
+# 129 takes a full tile), over short and long reductions, also beside one group of several full tiles.  With
+# f = 8192 and more fc2's forward and fc1's input gradient split their last round along K, so a short tile's
+# pieces meet: of fragments without rows, of unequal pieces, and beside a full tile's.
 FEW_ROW_CASES = [
     ("short-tiles", torch.bfloat16, 320, 192, [1, 15, 16, 17, 127, 128, 129, 0]),
-    ("short-split", torch.bfloat16, 2048, 2112, [1, 0, 16, 17, 64, 128, 33, 129]),
-    ("short-split-ragged-k", torch.bfloat16, 2112, 2496, [40]),
-    ("hot-group-split", torch.bfloat16, 2048, 2048, [600, 1] + [0] * 14),
+    ("short-k2048", torch.bfloat16, 2048, 2112, [1, 0, 16, 17, 64, 128, 33, 129]),
+    ("short-k2112", torch.bfloat16, 2112, 2496, [40]),
+    ("hot-group-k2048", torch.bfloat16, 2048, 2048, [600, 1] + [0] * 14),
+    ("short-split", torch.bfloat16, 256, 8192, [1, 0, 16, 17, 64, 128, 33, 129]),
+    ("short-split-ragged-k", torch.bfloat16, 320, 8256, [40]),
+    ("hot-group-split", torch.bfloat16, 256, 8192, [600, 1] + [0] * 14),
 ]
 
 
@@ -127,6 +131,37 @@ FEW_ROW_CASES = [
 @pytest.mark.parametrize("case", FEW_ROW_CASES, ids=[c[0] for c in FEW_ROW_CASES])
 def test_few_rows_per_group(case, act):
     test_grouped_expert_gemms(case, act)
+
+
+@pytest.mark.parametrize("act", ["swiglu", "gelu"])
+@pytest.mark.parametrize("h,f", [(2048, 2048), (4032, 3968)])
+def test_rows_keep_their_bits_in_any_batch(h, f, act):
+    """Reductions below 8192 are one chain over k, so a row's outputs are the same bits whatever rows share its
+    launch: alone in its group (short tiles), with 40 others a group, and in groups of more than a tile."""
+    dt, G, most = torch.bfloat16, 3, 300
+    F1 = 2 * f if act == "swiglu" else f
+    d = lambda *sh, seed, std: seeded(sh, seed, std, dt).to(DEV)  # noqa: E731
+    x, a, dy, hp, dh = (d(G, most, n, seed=i, std=1.0) for i, n in enumerate((h, f, h, F1, F1)))
+    w1 = [d(F1, h, seed=10 + g, std=0.05) for g in range(G)]
+    w2 = [d(h, f, seed=20 + g, std=0.05) for g in range(G)]
+    say(f"gemm rows in any batch h={h} f={f} {act}")
+    first = []
+    for n in (1, 41, most):
+        P = G * n
+        offs = torch.arange(0, P + 1, n, dtype=torch.int32, device=DEV)
+        xs, as_, dys, hps, dhs = ([t[:, :n].reshape(P, -1).contiguous()] * G for t in (x, a, dy, hp, dh))
+        outs = [torch.empty(P, c, dtype=dt, device=DEV) for c in (F1, f, h, F1, h, f)]
+        hpre, act_out, y, dhpre, dx, alone = ([t] * G for t in outs)
+        K.expert_fc1_fwd(xs, offs, True, P, w1, f, act, hpre, act_out)
+        K.expert_fc1_act(xs, offs, True, P, w1, f, act, alone)
+        K.expert_fc2_fwd(as_, offs, True, P, w2, y)
+        K.expert_fc2_bwd(dys, as_, hps, offs, True, P, w2, act, dhpre, None)
+        K.expert_fc1_bwd(dhs, xs, offs, True, P, w1, f, act, dx, None)
+        torch.cuda.synchronize()
+        first.append([t.view(G, n, -1)[:, 0].clone() for t in outs])
+    for other in first[1:]:
+        for name, p, q in zip(("hpre", "act", "y", "dhpre", "dx", "act alone"), first[0], other):
+            assert torch.equal(p, q), name
 
 
 # The generic kernel's edges: reductions and columns that end inside a stage, a quad and a 16-wide fragment
