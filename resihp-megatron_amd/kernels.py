@@ -102,16 +102,21 @@ def _distinct(ts):
     return out
 
 
+def _each(ts):
+    """The groups of a product for ``_need_cuda``: those of a stacked tensor one by one."""
+    return ts.unbind() if isinstance(ts, torch.Tensor) else ts
+
+
 def _need_cuda(*ts) -> torch.device:
-    """The HIP device of tensors, lists of tensors, Groups and Nones."""
+    """The HIP device of tensors, sequences of tensors, Groups and Nones."""
     flat = []
     for t in ts:
         if isinstance(t, Group):
             flat.append(t.ts[0])   # the others are alike
-        elif isinstance(t, (list, tuple)):
-            flat.extend(_distinct(t))
-        else:
+        elif t is None or isinstance(t, torch.Tensor):
             flat.append(t)
+        else:
+            flat.extend(_distinct(t))
     dev = None
     for t in flat:
         if t is None:
@@ -534,7 +539,7 @@ def _split_call(name: str, dev: torch.device, split: bool, *args) -> None:
 def expert_fc1_fwd(xs: list[torch.Tensor], offsets: torch.Tensor, rows_from_offsets: bool, rows_cap: int,
                    w1: list[torch.Tensor], f: int, act: str, hpre: list[torch.Tensor],
                    act_out: list[torch.Tensor], split: bool = True) -> None:
-    dev = _need_cuda(offsets, xs, w1, hpre, act_out)
+    dev = _need_cuda(offsets, _each(xs), _each(w1), _each(hpre), _each(act_out))
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     rows = _shared_rows(rows_from_offsets, rows_cap)
@@ -550,7 +555,7 @@ def expert_fc1_fwd(xs: list[torch.Tensor], offsets: torch.Tensor, rows_from_offs
 def expert_fc1_act(xs: list[torch.Tensor], offsets: torch.Tensor, rows_from_offsets: bool, rows_cap: int,
                    w1: list[torch.Tensor], f: int, act: str, act_out: list[torch.Tensor], split: bool = True) -> None:
     """expert_fc1_fwd where no backward follows: only the activation rows are written."""
-    dev = _need_cuda(offsets, xs, w1, act_out)
+    dev = _need_cuda(offsets, _each(xs), _each(w1), _each(act_out))
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     rows = _shared_rows(rows_from_offsets, rows_cap)
     _check_offsets(offsets, G)
@@ -563,7 +568,7 @@ def expert_fc1_act(xs: list[torch.Tensor], offsets: torch.Tensor, rows_from_offs
 
 def expert_fc2_fwd(acts: list[torch.Tensor], offsets: torch.Tensor, rows_from_offsets: bool, rows_cap: int,
                    w2: list[torch.Tensor], ys: list[torch.Tensor], split: bool = True) -> None:
-    dev = _need_cuda(offsets, acts, w2, ys)
+    dev = _need_cuda(offsets, _each(acts), _each(w2), _each(ys))
     G, dt, (h, f) = len(w2), w2[0].dtype, tuple(w2[0].shape)
     rows = _shared_rows(rows_from_offsets, rows_cap)
     _check_offsets(offsets, G)
@@ -580,7 +585,7 @@ def expert_fc2_bwd(dys: list[torch.Tensor], acts: list[torch.Tensor], hpres: lis
     """Input-gradient product into ``dhpre`` and weight gradient into ``dw2``; either may be None (not
     both), so the two independent products can run on two streams.  ``w2`` gives the shapes either way."""
     _expect(dhpre is not None or dw2 is not None, "expert_fc2_bwd: nothing to compute")
-    dev = _need_cuda(offsets, dys, acts, hpres, w2, dhpre, dw2)
+    dev = _need_cuda(offsets, *map(_each, (dys, acts, hpres, w2, dhpre, dw2)))
     G, dt, (h, f) = len(w2), w2[0].dtype, tuple(w2[0].shape)
     F1 = 2 * f if act == "swiglu" else f
     rows = _shared_rows(rows_from_offsets, rows_cap)
@@ -604,7 +609,7 @@ def expert_fc1_bwd(dhpre: list[torch.Tensor], xs: list[torch.Tensor], offsets: t
                    dxs: list[torch.Tensor] | None, dw1: list[torch.Tensor] | None, split: bool = True) -> None:
     """Input gradient into ``dxs`` and weight gradient into ``dw1``; either may be None (not both)."""
     _expect(bool(dxs) or dw1 is not None, "expert_fc1_bwd: nothing to compute")
-    dev = _need_cuda(offsets, dhpre, xs, w1, dxs, dw1)
+    dev = _need_cuda(offsets, *map(_each, (dhpre, xs, w1, dxs, dw1)))
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     rows = _shared_rows(rows_from_offsets, rows_cap)
@@ -630,7 +635,7 @@ def expert_fc1_fwd_gather(src: torch.Tensor, src_idx: torch.Tensor, offsets: tor
                           w1: list[torch.Tensor], f: int, act: str, hpre: torch.Tensor, act_out: torch.Tensor,
                           split: bool = True) -> None:
     """expert_fc1_fwd on rows gathered from ``src``: grouped row r is ``src[src_idx[r]]`` (no copy)."""
-    dev = _need_cuda(offsets, src, src_idx, w1, hpre, act_out)
+    dev = _need_cuda(offsets, src, src_idx, _each(w1), hpre, act_out)
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     _check_offsets(offsets, G)
@@ -646,7 +651,7 @@ def expert_fc1_fwd_gather(src: torch.Tensor, src_idx: torch.Tensor, offsets: tor
 def expert_fc2_fwd_scatter(act_in: torch.Tensor, offsets: torch.Tensor, rows_cap: int, w2: list[torch.Tensor],
                            y: torch.Tensor, y_idx: torch.Tensor, split: bool = True) -> None:
     """expert_fc2_fwd writing grouped row r to ``y[y_idx[r]]`` (no copy)."""
-    dev = _need_cuda(offsets, act_in, y, y_idx, w2)
+    dev = _need_cuda(offsets, act_in, y, y_idx, _each(w2))
     G, dt, (h, f) = len(w2), w2[0].dtype, tuple(w2[0].shape)
     _check_offsets(offsets, G)
     _check_map("y_idx", y_idx, rows_cap)
@@ -661,7 +666,7 @@ def expert_fc2_dgrad_gather(dy: torch.Tensor, dy_idx: torch.Tensor, offsets: tor
                             w2: list[torch.Tensor], act: str, hpre: torch.Tensor, dhpre: torch.Tensor,
                             split: bool = True) -> None:
     """The input-gradient product of expert_fc2_bwd on output-gradient rows ``dy[dy_idx[r]]`` (no copy)."""
-    dev = _need_cuda(offsets, dy, dy_idx, hpre, dhpre, w2)
+    dev = _need_cuda(offsets, dy, dy_idx, hpre, dhpre, _each(w2))
     G, dt, (h, f) = len(w2), w2[0].dtype, tuple(w2[0].shape)
     F1 = 2 * f if act == "swiglu" else f
     _check_offsets(offsets, G)
@@ -677,7 +682,7 @@ def expert_fc2_dgrad_gather(dy: torch.Tensor, dy_idx: torch.Tensor, offsets: tor
 def expert_fc1_dgrad_scatter(dhpre: torch.Tensor, offsets: torch.Tensor, rows_cap: int, w1: list[torch.Tensor],
                              f: int, act: str, dx: torch.Tensor, dx_idx: torch.Tensor, split: bool = True) -> None:
     """The input-gradient product of expert_fc1_bwd writing grouped row r to ``dx[dx_idx[r]]`` (no copy)."""
-    dev = _need_cuda(offsets, dhpre, dx, dx_idx, w1)
+    dev = _need_cuda(offsets, dhpre, dx, dx_idx, _each(w1))
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     _check_offsets(offsets, G)
@@ -694,7 +699,7 @@ def expert_fc1_dgrad_router(dhpre: list[torch.Tensor], offsets: torch.Tensor, ro
                             dxs: list[torch.Tensor], split: bool = True) -> None:
     """fc1's input gradient with the router term added per row: ``dxs[r] = dhpre[r] @ w1 + dl[perm[r]] *
     router_w[e0 + g]`` (then token_bwd runs without ``dl``).  Every expert of the layer must be local."""
-    dev = _need_cuda(offsets, router_w, perm, dl, dhpre, w1, dxs)
+    dev = _need_cuda(offsets, router_w, perm, dl, _each(dhpre), _each(w1), _each(dxs))
     G, dt, h = len(w1), w1[0].dtype, w1[0].shape[1]
     F1 = 2 * f if act == "swiglu" else f
     _check_offsets(offsets, G)

@@ -526,3 +526,34 @@ def test_fc1_dgrad_router_term(dtype, h, f, counts, e0):
     # the router term is really there: without it the rows differ by far more than the rounding
     bare = torch.cat([dh[o[i]:o[i + 1]].double() @ w1[i].double() for i in range(G)])
     assert rel_err(bare, ref) > 1e-2
+
+
+def test_groups_in_any_sequence():
+    """The groups of a product may be any sequence of tensors: a list, a ParameterList, a stack whose groups
+    are contiguous though the stack is not.  A group that is not contiguous is refused in each."""
+    dt, h, f, M = torch.bfloat16, 128, 64, 9
+    offs = torch.tensor([0, 4, M], dtype=torch.int32, device=DEV)
+    d = lambda *sh, seed, std: seeded(sh, seed, std, dt).to(DEV)  # noqa: E731
+    x, w1, w2 = d(M, h, seed=1, std=1.0), d(4, 2 * f, h, seed=2, std=0.05)[::2], d(4, h, f, seed=3, std=0.05)[::2]
+    dy = d(M, h, seed=4, std=1.0)
+    forms = [list, lambda t: t, tuple,
+             lambda t: torch.nn.ParameterList(torch.nn.Parameter(g, requires_grad=False) for g in t)]
+    say("gemm groups in any sequence")
+    results = []
+    for form in forms:
+        hp, a, y, dh, dx = (torch.empty(M, n, dtype=dt, device=DEV) for n in (2 * f, f, h, 2 * f, h))
+        dw1, dw2 = (torch.zeros(4, *t.shape[1:], dtype=dt, device=DEV)[::2] for t in (w1, w2))
+        K.expert_fc1_fwd([x] * 2, offs, True, M, form(w1), f, "swiglu", [hp] * 2, [a] * 2)
+        K.expert_fc2_fwd([a] * 2, offs, True, M, form(w2), [y] * 2)
+        K.expert_fc2_bwd([dy] * 2, [a] * 2, [hp] * 2, offs, True, M, form(w2), "swiglu", [dh] * 2, list(dw2))
+        K.expert_fc1_bwd([dh] * 2, [x] * 2, offs, True, M, form(w1), f, "swiglu", [dx] * 2, list(dw1))
+        results.append([t.clone() for t in (hp, a, y, dh, dx, dw1, dw2)])
+    torch.cuda.synchronize()
+    assert results[0][6].abs().sum() > 0
+    for other in results[1:]:
+        for p, q in zip(results[0], other):
+            assert torch.equal(p, q)
+    bad = torch.empty(2, h, 2 * f, dtype=dt, device=DEV).transpose(1, 2)
+    for form in forms:
+        with pytest.raises(RuntimeError, match="contiguous"):
+            K.expert_fc1_fwd([x] * 2, offs, True, M, form(bad), f, "swiglu", [hp] * 2, [a] * 2)
