@@ -66,6 +66,10 @@ const char* rhp_last_error(void);
  * (segments of min(256,h) elements, each one fused-multiply-add chain, summed
  * left to right) so that results are reproducible bit for bit.
  * Requires h % 8 == 0, h % min(256,h) == 0, 1 <= k <= min(E, 16), E <= 1024.
+ * Any token count.  Float32 and bfloat16 tokens of up to 511 and 1023 experts
+ * (odd E, or E + 1, plus 2 k) take any h with E h 4 bytes and 16 token rows
+ * below 2 GiB; other sizes need 4 ((h / min(256,h) + 1) E sizeof(r_dtype) + 4 k)
+ * bytes within 48 KB.
  */
 int rhp_route(const void* x, int x_dtype, const void* router_w, int r_dtype, const void* bias, int64_t T,
               int h, int E, int k, int score, int normalize, double scale, void* logits, int32_t* topi,

@@ -830,17 +830,31 @@ int launch_route_mfma(const void* x, const void* w, const void* bias, int64_t T,
     return check_launch("route_mfma_kernel");
 }
 
-// Sizes of bfloat16 tokens that are taken whatever the per-thread kernel's LDS limit: those whose
-// logits and, with few experts, segment sums of one block of tokens fit in 64 KB.
-bool bf16_route_fits(int64_t T, int h, int E, int k) {
-    const int S = h / std::min(256, h), ec = E >= 64 ? 16 : 8, n_ec = (E + ec - 1) / ec;
-    const size_t tok = (T + 63) / 64 < device_cus() ? 32 : 64;
-    return tok * (E + k) * 4 + (n_ec >= S ? 0 : static_cast<size_t>(S) * ec * tok * 4) <= 64 * 1024;
+// Sizes a route_mfma_kernel takes, whatever the token count: its block's logits and selection fit beside the
+// staging buffers, and the byte offsets of the router's and of a block's token rows in 31 bits.
+template <class XT, int TI, int NB> bool rt_takes(int h, int E, int k) {
+    constexpr int64_t limit = int64_t(1) << 31;
+    return rt_lds(16 * TI, E, k) <= rt_room<XT, TI, NB>() && static_cast<int64_t>(E) * h * 4 < limit &&
+           int64_t(16) * TI * h * static_cast<int64_t>(sizeof(XT)) < limit;
 }
 
 template <class XT, class AT>
 int launch_route(const void* x, const void* w, const void* bias, int64_t T, int h, int E, int k, int score,
                  int normalize, double scale, void* logits, int32_t* topi, void* gates, hipStream_t stream) {
+    if constexpr (std::is_same<AT, float>::value) {
+        int (*mfma)(const void*, const void*, const void*, int64_t, int, int, int, int, int, double, void*, int32_t*,
+                    void*, hipStream_t) = nullptr;
+        if constexpr (std::is_same<XT, bf16>::value) {
+            if (T >= kRtWideTokens && rt_takes<XT, 2, 2>(h, E, k)) mfma = launch_route_mfma<XT, 2, 2>;
+            else if (rt_takes<XT, 1, 3>(h, E, k)) mfma = launch_route_mfma<XT, 1, 3>;
+        }
+        if (!mfma && rt_takes<XT, 1, 2>(h, E, k)) mfma = launch_route_mfma<XT, 1, 2>;
+        if (mfma) {
+            if (T == 0) return 0;
+            return mfma(x, w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates, stream);
+        }
+    }
+    // float64 tokens, and more experts than the kernel above holds (E + 2 k past 1023 in bfloat16, 511 in float32).
     RouteShape rs;
     rs.seg = std::min(256, h);
     rs.S = h / rs.seg;
@@ -854,22 +868,8 @@ int launch_route(const void* x, const void* w, const void* bias, int64_t T, int 
     rs.ntg = ntg;
     rs.tb = ntg * kTpt;
     const size_t smem = static_cast<size_t>(rs.tb) * per_token;
-    constexpr bool bf = std::is_same<XT, bf16>::value;
-    RHP_REQUIRE(smem <= 48 * 1024 || (bf && bf16_route_fits(T, h, E, k)),
-                "rhp_route: hidden size x experts too large for one routing block");
+    RHP_REQUIRE(smem <= 48 * 1024, "rhp_route: hidden size x experts too large for one routing block");
     if (T == 0) return 0;
-    if constexpr (std::is_same<AT, float>::value) {
-        if (static_cast<int64_t>(E) * h * 4 < (int64_t(1) << 31)) {
-            if constexpr (bf) {
-                if (T >= kRtWideTokens && rt_lds(32, E, k) <= rt_room<XT, 2, 2>())
-                    return launch_route_mfma<XT, 2, 2>(x, w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates, stream);
-                if (rt_lds(16, E, k) <= rt_room<XT, 1, 3>())
-                    return launch_route_mfma<XT, 1, 3>(x, w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates, stream);
-            }
-            if (rt_lds(16, E, k) <= rt_room<XT, 1, 2>())
-                return launch_route_mfma<XT, 1, 2>(x, w, bias, T, h, E, k, score, normalize, scale, logits, topi, gates, stream);
-        }
-    }
     const int64_t blocks = (T + rs.tb - 1) / rs.tb;
     hipLaunchKernelGGL((route_kernel<XT, AT>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads),
                        smem + static_cast<size_t>(rs.tb) * k * sizeof(AT), stream,

@@ -44,6 +44,13 @@ def test_abi_version_and_enums_match_header():
     (dict(T=4, h=60, E=4, k=2, xd=C.BF16, rd=C.F32), "multiple of 8"),
     # float64 model with a float32 router
     (dict(T=4, h=64, E=4, k=2, xd=C.F64, rd=C.F32), "float64 router"),
+    # a block's token rows, and the router weights, past 31-bit offsets
+    (dict(T=4, h=1 << 26, E=1, k=1, xd=C.BF16, rd=C.F32), "too large"),
+    (dict(T=0, h=1 << 25, E=1, k=1, xd=C.F32, rd=C.F32), "too large"),
+    (dict(T=4, h=1 << 21, E=256, k=1, xd=C.BF16, rd=C.F32), "too large"),
+    # float64 tokens, and more experts than the matrix-core kernel holds: a block's segment sums past 48 KB
+    (dict(T=4, h=4096, E=256, k=2, xd=C.F64, rd=C.F64), "too large"),
+    (dict(T=4, h=512, E=1024, k=8, xd=C.BF16, rd=C.F32), "too large"),
 ])
 def test_route_rejects_bad_arguments(args, msg):
     fake = ctypes.c_void_p(4096)   # never dereferenced: validation fails first

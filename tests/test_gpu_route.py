@@ -88,6 +88,24 @@ def test_route_kernel_edges(case):
     test_route_bit_exact(case)
 
 
+@pytest.mark.parametrize("T,h,E,k,xdt", [(16321, 4096, 320, 8, torch.bfloat16), (16320, 4096, 320, 8, torch.bfloat16),
+                                         (37, 4096, 256, 8, torch.float32), (70, 16384, 500, 4, torch.bfloat16)])
+def test_route_takes_any_token_count(T, h, E, k, xdt):
+    """Sizes the matrix-core kernel's LDS holds are taken whatever the token count, float32 tokens too."""
+    n = min(T, 37)
+    base, w = seeded((n, h), 7, 1.0, xdt), seeded((E, h), 8, 0.02, torch.float32)
+    x = base.repeat(T // n + 1, 1)[:T]
+    say(f"route any T={T} h={h} E={E} k={k} {xdt}")
+    logits, topi, gates = K.route(x.to(DEV), w.to(DEV), None, k, "softmax", True, 1.0)
+    torch.cuda.synchronize()
+    ref_logits = R.router_logits(host_x(base), w.numpy(), x_kind(xdt))
+    ref_topi, ref_gates = R.topk(ref_logits, k)
+    rows = np.arange(T) % n
+    assert np.array_equal(logits.cpu().numpy().view(np.int32), ref_logits.view(np.int32)[rows])
+    assert np.array_equal(topi.cpu().numpy(), ref_topi[rows])
+    assert np.array_equal(gates.cpu().numpy().view(np.int32), ref_gates.view(np.int32)[rows])
+
+
 def test_route_ties_over_candidates():
     # 130 experts in equal pairs two lanes' candidates apart: the lower id of each pair comes first.
     T, h, E, k = 37, 256, 130, 8
