@@ -27,14 +27,13 @@ ROUTE_CASES = [
     ("ep128-zipf", 8192, 2048, 128, 8, torch.bfloat16, "softmax", "zipf", 0.02),
     ("reference-default", 48, 8, 6, 2, torch.float64, "softmax", None, 0.35),
     ("odd-e", 333, 256, 5, 3, torch.bfloat16, "sigmoid", None, 0.05),
-    # bfloat16 kernel edges: a hidden size below one 256-element segment (ragged last 64-element group),
-    # expert counts that are not a multiple of the 8- or 16-expert groups, 32 segments (waves loop over
-    # segments), the expert-parallel mode (at least as many expert groups as segments), and more experts
-    # than its LDS holds (generic kernel)
+    # a hidden size below one 256-element segment (ragged last 16-element batch), expert counts that are not a
+    # multiple of 16, 32 segments, more expert tiles than waves, and more experts than the three-batch staging
+    # of 16-token blocks leaves room for
     ("bf16-h200-e20", 130, 200, 20, 4, torch.bfloat16, "softmax", "normal", 0.05),
     ("bf16-h8192-e72", 100, 8192, 72, 6, torch.bfloat16, "sigmoid", "normal", 0.02),
-    ("bf16-expert-mode-e200", 150, 1024, 200, 8, torch.bfloat16, "softmax", "zipf", 0.02),
-    ("bf16-e300-generic", 70, 256, 300, 4, torch.bfloat16, "softmax", None, 0.05),
+    ("bf16-e200", 150, 1024, 200, 8, torch.bfloat16, "softmax", "zipf", 0.02),
+    ("bf16-e300", 70, 256, 300, 4, torch.bfloat16, "softmax", None, 0.05),
 ]
 
 
@@ -68,12 +67,22 @@ def test_route_bit_exact(case):
 
 # Edges of the matrix-core kernel: one token, a ragged last 16-token tile at both block sizes (16 and, from
 # 8192 bf16 tokens, 32), segment counts that are not a multiple of four, more segment quads than waves (the
-# sums continue over rounds), one expert, expert tiles over several rounds, and the LDS limits of its buffers.
+# sums continue over rounds), one expert, expert tiles over several rounds, and the LDS limits of its buffers:
+# the last size of each (E odd or one less, plus 2 k: 255 for 32-token blocks, 1023 in bfloat16, 511 in float32)
+# and the first past it, which takes 16-token blocks and, "per-thread", the kernel of a thread per chain.
 EDGE_CASES = [
     ("one-token", 1, 4096, 8, 2, torch.bfloat16, "softmax", None, 0.02),
     ("t8191", 8191, 256, 16, 2, torch.bfloat16, "softmax", None, 0.05),
     ("t8197-wide", 8197, 512, 33, 4, torch.bfloat16, "sigmoid", "normal", 0.05),
-    ("t8192-wide-e250", 8192, 256, 250, 8, torch.bfloat16, "softmax", "zipf", 0.05),
+    ("t8192-wide-e239", 8192, 256, 239, 8, torch.bfloat16, "softmax", "zipf", 0.05),
+    ("t8192-e240", 8192, 256, 240, 8, torch.bfloat16, "softmax", "zipf", 0.05),
+    ("t8192-e250", 8192, 256, 250, 8, torch.bfloat16, "softmax", "zipf", 0.05),
+    ("e1007", 70, 256, 1007, 8, torch.bfloat16, "sigmoid", "normal", 0.05),
+    ("e1008-per-thread", 70, 256, 1008, 8, torch.bfloat16, "sigmoid", "normal", 0.05),
+    ("e1024-per-thread", 71, 256, 1024, 8, torch.bfloat16, "softmax", "zipf", 0.05),
+    ("f32-e495", 37, 256, 495, 8, torch.float32, "softmax", "normal", 0.05),
+    ("f32-e496-per-thread", 37, 256, 496, 8, torch.float32, "softmax", "normal", 0.05),
+    ("f32-e600-h512-per-thread", 21, 512, 600, 4, torch.float32, "sigmoid", "normal", 0.05),
     ("five-segments", 77, 1280, 17, 3, torch.bfloat16, "softmax", None, 0.03),
     ("sixteen-quads", 40, 16384, 24, 4, torch.bfloat16, "softmax", None, 0.01),
     ("h8-e1", 50, 8, 1, 1, torch.bfloat16, "softmax", None, 0.3),
@@ -106,16 +115,17 @@ def test_route_takes_any_token_count(T, h, E, k, xdt):
     assert np.array_equal(gates.cpu().numpy().view(np.int32), ref_gates.view(np.int32)[rows])
 
 
-def test_route_ties_over_candidates():
-    # 130 experts in equal pairs two lanes' candidates apart: the lower id of each pair comes first.
-    T, h, E, k = 37, 256, 130, 8
-    x = seeded((T, h), 5, 1.0, torch.bfloat16)
+@pytest.mark.parametrize("E,xdt", [(130, torch.bfloat16), (1024, torch.bfloat16), (600, torch.float32)])
+def test_route_ties_over_candidates(E, xdt):
+    # Experts in equal pairs two lanes' candidates apart, in both kernels: the lower id of each pair comes first.
+    T, h, k = 37, 256, 8
+    x = seeded((T, h), 5, 1.0, xdt)
     w = seeded((E, h), 6, 0.05, torch.float32)
     w[64:128] = w[0:64]
     w[3] = w[2]
-    say("route ties over 130 experts")
+    say(f"route ties over {E} experts {xdt}")
     logits, topi, gates = K.route(x.to(DEV), w.to(DEV), None, k, "softmax", True, 1.0)
-    ref_logits = R.router_logits(host_x(x), w.numpy(), "bf16")
+    ref_logits = R.router_logits(host_x(x), w.numpy(), x_kind(xdt))
     ref_topi, ref_gates = R.topk(ref_logits, k)
     assert np.array_equal(topi.cpu().numpy(), ref_topi)
     assert np.array_equal(gates.cpu().numpy().view(np.uint8), ref_gates.view(np.uint8))
