@@ -76,6 +76,17 @@ def test_dispatch_and_gemm_reject_bad_arguments():
     with pytest.raises(RuntimeError, match="split workspace"):
         C.call("rhp_expert_fc1_bwd", 1, fake, 1, 0, C.BF16, C.ACT_SWIGLU, 64, 64, ptrs, ptrs, ptrs, ptrs, ptrs,
                ctypes.c_void_p(4097), C.lib().rhp_expert_split_workspace_bytes(), None)
+    null = C.ptr_array([0])
+    for x, w, out, msg in ((null, ptrs, ptrs, "null pointer"), (ptrs, null, ptrs, "null pointer"),
+                           (ptrs, ptrs, null, "null pointer"), (C.ptr_array([4104]), ptrs, ptrs, "16-byte aligned")):
+        with pytest.raises(RuntimeError, match=msg):
+            C.call("rhp_expert_fc1_act", 1, fake, 1, 0, C.BF16, C.ACT_SWIGLU, 64, 64, x, w, out, None, 0, None)
+    with pytest.raises(RuntimeError, match="split workspace"):
+        C.call("rhp_expert_fc1_act", 1, fake, 1, 0, C.BF16, C.ACT_SWIGLU, 64, 64, ptrs, ptrs, ptrs, fake, 1024, None)
+    for hpre in (None, null):
+        with pytest.raises(RuntimeError, match="null pointer"):
+            C.call("rhp_expert_fc1_fwd", 1, fake, 1, 0, C.BF16, C.ACT_SWIGLU, 64, 64, ptrs, ptrs, hpre, ptrs, None, 0,
+                   None)
     with pytest.raises(RuntimeError, match="at most 8 shared"):
         C.call("rhp_combine", fake, fake, fake, C.F32, fake, fake, ptrs, 9, C.BF16, 4, 64, 2, fake, None)
 

@@ -237,14 +237,14 @@ def test_generic_kernel_unaligned_operands(dt):
 
 
 @pytest.mark.parametrize("T", [200, 513, 2048])
-def test_per_group_buffers_shared_expert_mode(T):
+def test_per_group_buffers_shared_expert_mode(T, f=128):
     """rows_from_offsets = 0: each group reads and writes its own buffer from row 0 (shared experts).
 
     The grid must cover every group's row tiles: with two groups of T rows each that is 2 ceil(T / 256)
     row tiles, more than ceil(T / 256) + 2 once T exceeds 512 (2048: 16 against 10).  Every output and
     gradient of both groups is checked, forward and backward.
     """
-    dt, h, f, S, act = torch.bfloat16, 256, 128, 2, "swiglu"
+    dt, h, S, act = torch.bfloat16, 256, 2, "swiglu"
     offs = (torch.arange(S + 1, dtype=torch.int32) * T).to(DEV)
     xs = [seeded((T, h), 5 + s, 1.0, dt) for s in range(S)]
     w1 = [seeded((2 * f, h), 50 + s, 0.05, dt) for s in range(S)]
@@ -252,7 +252,7 @@ def test_per_group_buffers_shared_expert_mode(T):
     dys = [seeded((T, h), 70 + s, 1.0, dt) for s in range(S)]
     d = lambda ts: [t.to(DEV) for t in ts]  # noqa: E731
     xs_d, w1_d, w2_d, dys_d = d(xs), d(w1), d(w2), d(dys)
-    say(f"gemm shared-expert buffers T={T}")
+    say(f"gemm shared-expert buffers T={T} f={f}")
     hs = [torch.empty(T, 2 * f, dtype=dt, device=DEV) for _ in range(S)]
     as_ = [torch.empty(T, f, dtype=dt, device=DEV) for _ in range(S)]
     ys = [torch.empty(T, h, dtype=dt, device=DEV) for _ in range(S)]
@@ -276,6 +276,12 @@ def test_per_group_buffers_shared_expert_mode(T):
         assert rel_err(dw2[s], dy64.t() @ a64) <= 1e-2, ("dw2", s)
         assert rel_err(dx[s], dh64 @ c64(w1[s])) <= 1e-2, ("dx", s)
         assert rel_err(dw1[s], dh64.t() @ x64) <= 1e-2, ("dw1", s)
+
+
+@pytest.mark.parametrize("T", [1, 37, 64, 128])
+def test_per_group_buffers_of_few_rows(T):
+    """Short tiles of groups with a buffer each, their last round split along K (reductions of 8192 and 16384)."""
+    test_per_group_buffers_shared_expert_mode(T, f=8192)
 
 
 def test_gemm_deterministic():

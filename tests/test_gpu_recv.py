@@ -112,14 +112,14 @@ def _map_case(counts, src_rows, seed, invalid):
                                                (torch.float32, 128, 64, True)],
                          ids=["bf16-mfma", "bf16-mfma-ep128-dims-bad-idx", "bf16-mfma-k-split", "bf16-generic",
                               "f32-generic"])
-def test_row_map_products_equal_gather_then_product(dtype, h, f, invalid):
+def test_row_map_products_equal_gather_then_product(dtype, h, f, invalid, counts=None):
     """The four products on received rows (gathered inputs, scattered outputs) equal rhp_gather_rows
     followed by the plain product, bit for bit, on both kernels: ragged groups (one empty), distinct
     received rows in random order, indices outside the buffer (zero rows in, rows dropped out), and
     buffer rows that no index names (left untouched).  With f = 4096 fc1's input-gradient product
     reduces over 8192 and its last round is split along K (the scatter then runs in the epilogue of
     the piece that finishes last)."""
-    counts = [300, 0, 517, 64, 1029] if dtype == torch.bfloat16 and h >= 256 else [33, 0, 70, 5]
+    counts = counts or ([300, 0, 517, 64, 1029] if dtype == torch.bfloat16 and h >= 256 else [33, 0, 70, 5])
     src_rows = int(sum(counts)) + 41
     offsets, idx, P = _map_case(counts, src_rows, h + f, invalid)
     G = len(counts)
@@ -166,6 +166,13 @@ def test_row_map_products_equal_gather_then_product(dtype, h, f, invalid):
         assert torch.equal(out[~named], sentinel[~named])
     if invalid:
         assert not bool(ok.all()) and bool((xs[~ok] == 0).all())
+
+
+@pytest.mark.parametrize("h,f,counts", [(2048, 2048, [1, 0, 17, 64, 129]), (256, 8192, [1, 0, 17, 64, 129]),
+                                        (320, 4160, [40, 128])], ids=["k2048", "k-split", "k-split-ragged"])
+def test_row_map_products_of_few_rows(h, f, counts):
+    """The same on short tiles; from f = 4096 and 8192 fc1's input gradient and fc2's forward are split along K."""
+    test_row_map_products_equal_gather_then_product(torch.bfloat16, h, f, True, counts)
 
 
 def test_row_map_products_reject_bad_maps():
