@@ -38,9 +38,10 @@ constexpr int kAdamThreads = 256;
 // small blocks that come and go keep its reads and writes mixed.
 // 1.41 G bfloat16 parameters (14 bytes each, 256 threads a block): 4 groups a
 // thread with ordinary accesses 3664 us, 5.39 TB/s; non-temporal 3479; 2
-// groups 3487; 1 group 3305, 5.97 TB/s (ordinary accesses 3573).  Cutting a
-// quarter of the instructions (shorter exact square root and divisions)
-// changed none of these by more than 2 %, so the plain forms stay.
+// groups 3487; 1 group 3305, 5.97 TB/s (ordinary accesses 3573), all on one
+// card; others run the last in 3370-3420 us, 5.8 TB/s.  Cutting a quarter of
+// the instructions (shorter exact square root and divisions) changed none of
+// these by more than 2 %, so the plain forms stay.
 // Wider types take as many bytes, not as many elements, so that a wave's
 // access is whole lines: 8.6 M float32 parameters 46.6 us with 8 a thread, 40.2.
 template <class S> constexpr int kAdamElems = 16 / static_cast<int>(sizeof(S));

@@ -19,9 +19,10 @@
 // read with ds_read_b128; operands stored with K as the slow dimension are read
 // with gfx950's transposing LDS load (details at the kernel).
 //
-// Work unit: a 256 x 256 output tile.  Tiles are ordered group-major, then by
-// output column block, then by row block, and block ids are remapped so each
-// XCD runs a contiguous range of that order.
+// Work unit: a 256 x 256 output tile, or one of 128 rows where a group has no
+// more.  Tiles are ordered group-major, then by output column block, then by
+// row block, and block ids are remapped so each XCD runs a contiguous range of
+// that order.
 #include <type_traits>
 #include <vector>
 
@@ -669,8 +670,8 @@ __global__ __launch_bounds__(64 * NW) void gg_bf16_kernel(Params p) {
     if (find_tile<MODE>(p, x_per_tile<EPI>(), kTile, blockIdx.x, &t) != kTileOk) return;
     if constexpr (MODE != kWgrad) {
         // Only groups that have no full tile: they are bound by the weights' way to the CUs.  At the end of a
-        // larger group (or beside other full tiles) the GPU is at its power limit, where the idle waves cost
-        // nothing and the short tile gains nothing: a 1500-token Mixtral forward ran 3 % slower with it.
+        // larger group the short tile, which reads 12 fragments from LDS for 32 MFMAs against a full one's 16
+        // for 64, gains nothing: a 1500-token Mixtral forward ran 3 % slower with it.
         if (__builtin_amdgcn_readfirstlane(t.y_lim + t.y0) <= kTile / 2) {
             gg_bf16_short_tile<MODE, EPI, MAP>(p, t, lds);
             return;
